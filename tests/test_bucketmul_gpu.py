@@ -365,6 +365,20 @@ def test_narrow_and_ragged_columns(O, ctx, out_dim):
     check_against_oracle(O, ctx, b, s, p, x, 0.25)
 
 
+@pytest.mark.parametrize("out_dim", [16, 112, 1040, 1152 + 16])
+@pytest.mark.parametrize("rows", [65536, 65536 - 7])
+def test_unaligned_rows_to_the_last(O, iam, ctx, out_dim, rows):
+    """Columns that are no multiple of 8 (1, 7, 65 and 73 buckets): every row
+    selected, so the wide loads run up to the matrix's last row (whole and
+    partial last input), in the split call and in the two one-launch calls."""
+    b, s, p = make_matrix(O, out_dim, 4096, tid=8)
+    x = O.gen_f32(0, 9, 4096, 0.0, 1.0)
+    x[-2:] = (3.0, -4.0)
+    for kw in (dict(split=True), dict(split=False), dict(fused=iam)):
+        y, oy, cut, S = check_against_oracle(O, ctx, b[:rows], s[:rows], p, x, 1.0, in_size=4096, expert_rows=rows, **kw)
+        assert S > 0.99 * rows
+
+
 def test_in_size_skips_rows(O, ctx):
     b, s, p = make_matrix(O, 256, 4096, tid=13)
     x = O.gen_f32(0, 14, 4096, 0.0, 1.0)
