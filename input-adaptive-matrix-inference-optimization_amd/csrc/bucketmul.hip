@@ -1558,7 +1558,8 @@ int walk_group(Ctx* c, const WalkGroup& g)
 
 // The standalone walk of the n matrices recorded in slots 0..n-1: the
 // slots' scratch, fp32 outputs stored by the tiles' last workgroups.
-static int walk_slots(Ctx* c, int n, const MatOp* ops, int in_mode, const float* h, const uint16_t* gain, float eps)
+static int walk_slots(Ctx* c, int n, const MatOp* ops, int in_mode, const float* h, const uint16_t* gain, float eps,
+                      bool hints)
 {
     WalkGroup g;
     g.n = n;
@@ -1601,7 +1602,7 @@ static int walk_slots(Ctx* c, int n, const MatOp* ops, int in_mode, const float*
         wm.in_size = s.in_size;
         wm.x = s.x;
         wm.cutoff = s.cutoff;
-        wm.hint = c->hints && in_mode != kInCutoff ? s.cutoff + 2 : nullptr;
+        wm.hint = hints && c->hints ? s.cutoff + 2 : nullptr;
         wm.slice_count = s.slice_count;
         wm.acc = s.acc;
         wm.tile_ctr = s.tile_ctr;
@@ -1610,7 +1611,25 @@ static int walk_slots(Ctx* c, int n, const MatOp* ops, int in_mode, const float*
     return walk_group(c, g);
 }
 
-int bucketmul_walk(Ctx* c, int n, const MatOp* ops) { return walk_slots(c, n, ops, kInCutoff, nullptr, nullptr, 0.0f); }
+int bucketmul_walk(Ctx* c, int n, const MatOp* ops)
+{
+    return walk_slots(c, n, ops, kInCutoff, nullptr, nullptr, 0.0f, false);
+}
+
+// A whole product (or up to 3, each with its own x) of the full and multi
+// calls in one launch: every walk workgroup runs the cutoff search of its
+// matrix itself (unhinted: these calls have no previous cutoff to start
+// from) instead of waiting for a search launch of one workgroup per matrix.
+// The search inside the walk costs it about 3.5 us; the launch it replaces
+// took 6-8 us plus the gap between the two (1024 x 4096 at effort 0.25: 18.7
+// us a call before, 15.8 now; a 4096-wide layer of four such calls at effort
+// 0.25: 102.5 -> 85.4 us).
+static int bucketmul_whole(Ctx* c, int n, const MatOp* ops, int expert_no, float effort)
+{
+    CutoffArgs args{};
+    IAM_TRY(record_slots(c, n, ops, expert_no, effort, args));
+    return walk_slots(c, n, ops, kInX, nullptr, nullptr, 0.0f, false);
+}
 
 // One matrix group in one launch: every workgroup computes the input (x, or
 // the norm of h written to x) and the cutoff itself.  A norm input of other
@@ -1635,7 +1654,7 @@ int bucketmul_fused(Ctx* c, int n, const MatOp* ops, int expert_no, float effort
             in_mode = kInX;
         }
     }
-    return walk_slots(c, n, ops, in_mode, h, gain, eps);
+    return walk_slots(c, n, ops, in_mode, h, gain, eps, true);
 }
 
 __global__ void k_stats_compact(const uint16_t* __restrict__ s, size_t rows, int stride, int ch,
@@ -1701,8 +1720,7 @@ int iam_bucketmul_full(iam_ctx* c, const float* x, const uint16_t* stats, const 
     op.in_size = in_size;
     op.y = y;
     IAM_REQUIRE(y, "full: null y");
-    IAM_TRY(bucketmul_dispatch(c, 1, &op, expert_no, effort));
-    return bucketmul_walk(c, 1, &op);
+    return bucketmul_whole(c, 1, &op, expert_no, effort);
 }
 
 int iam_bucketmul_multi(iam_ctx* c, int n, const iam_bucket_matrix* mats, const float* const* xs,
@@ -1718,8 +1736,7 @@ int iam_bucketmul_multi(iam_ctx* c, int n, const iam_bucket_matrix* mats, const 
         ops[i].y = ys[i];
         IAM_REQUIRE(ys[i] && mats[i].buckets, "multi: null y/buckets");
     }
-    IAM_TRY(bucketmul_dispatch(c, n, ops, expert_no, effort));
-    return bucketmul_walk(c, n, ops);
+    return bucketmul_whole(c, n, ops, expert_no, effort);
 }
 
 int iam_bucketmul_fused(iam_ctx* c, int n, const iam_bucket_matrix* mats, float* x, int in_size,
