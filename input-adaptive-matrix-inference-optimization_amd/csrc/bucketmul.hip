@@ -315,17 +315,6 @@ __global__ __launch_bounds__(kCutThreads) void k_dispatch(DispatchDesc d)
 }
 
 // ----------------------------------------------------------------- walk ---
-// Blocks are dealt to the 8 XCDs round robin (block b -> XCD b % 8).  Remap
-// so that consecutive work items (the column tiles of one row slice, which
-// read the same stats, inputs and neighbouring lines of the same rows) land
-// on the same XCD and share its L2.
-__device__ __forceinline__ int xcd_remap(int b, int nblocks)
-{
-    const int q = nblocks >> 3, r = nblocks & 7;
-    const int xcd = b & 7, idx = b >> 3;
-    return xcd < r ? xcd * (q + 1) + idx : r * (q + 1) + (xcd - r) * q + idx;
-}
-
 // 16 bytes of the weight stream, loaded non-temporally: read once per
 // launch, the rows would otherwise evict the small vectors every launch
 // reads first (inputs, probes, gains, stats, the KV cache) from L2 and the

@@ -18,6 +18,7 @@
 
 #include "internal.h"
 #include "layer_ops.h"
+#include "wave.h"
 
 namespace iam {
 
@@ -70,130 +71,287 @@ __global__ void k_gen_f32(uint64_t key, size_t count, double mean, double sigma,
 
 __device__ __forceinline__ float h2f(uint16_t b) { return __half2float(__ushort_as_half(b)); }
 
-// probes: one thread per input column, float32 sum in j order
-__global__ void k_probes(const uint16_t* __restrict__ W, int out_dim, int in_dim, uint16_t* __restrict__ probes)
+// ------------------------------------------------------------ bucketizer ---
+// One pass over W.  Workgroup g owns the 16 inputs (columns of W) 16g ..
+// 16g + 15 and walks the buckets in order, 64 at a time; 8 waves sort and
+// emit, a ninth adds the probes.  Per chunk of 64 buckets:
+//   sort    thread (column pair, bucket) holds 2 columns x 16 rows (its loads
+//           for the next chunk go out before the barrier), sorts each
+//           column's 16 keys by a network, and stores them by rank in LDS
+//           (s_key) and, in row order, for the probes (s_raw)
+//   emit    the rows' codes (lane = bucket: 128 consecutive bytes a wave
+//           store), and the rows' sums for the stats: 8 lanes per row, one
+//           per accumulator of numpy's 8-way unrolled block
+//   probes  the ninth wave adds each column's |w| in row order, the first
+//           half of the chunk during its emit, the second during the next
+//           sort
+// 14336 x 4096, with the compact stats: 1420 us a call for three passes (the
+// probes with one load chain per column, a sort whose 2-byte stores lay 2 * nb
+// bytes apart, then the sums re-reading W through the codes' positions), now
+// 142 us; 2000 x 300: 32.9 -> 10.3 us.  W and the codes once at the part's
+// copy rate are 47 us.  What bounds it now: the phases of the one workgroup a
+// CU holds follow each other (sorting, emitting and adding are about 50 us of
+// vector instructions, the waits between them as much again), and the probes'
+// chain of dependent adds takes issue slots from one SIMD (without it: 106 us).
+// 8 columns per workgroup, two to a CU: 226 us.
+constexpr int kBkInputs = 16;               // columns of W per workgroup
+constexpr int kBkChunk = 64;                // buckets per chunk
+constexpr int kBkWorkers = 512;             // sorting threads (8 column pairs x 64 buckets)
+constexpr int kBkThreads = kBkWorkers + 64; // and the wave of the probes
+constexpr int kBkKeyStride = kBkChunk + 4;  // words per (rank, column): 8 column pairs x 8 buckets on 64 banks
+constexpr int kBkRawStride = kBkChunk * 16 + 8;   // halves per column: 16-byte reads on disjoint banks
+constexpr int kBkDepth = 24;                // levels of the pairwise tree: blocks of at least 64, up to 2^27 buckets
+
+// One element's sort key: |w| (15 bits), then the earlier position first,
+// with the sign along: descending keys are the reference's order (|w|
+// descending, ties in original order), and each key holds its code and its
+// |w|.  A NaN sorts by its bits, above infinity.
+__device__ __forceinline__ uint32_t bucket_key(uint32_t w, int p)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= in_dim) return;
-    float acc = 0.0f;
-    int j = 0;
-    for (; j + 8 <= out_dim; j += 8) {
-        uint16_t v[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) v[u] = W[(size_t)(j + u) * in_dim + i];
-#pragma unroll
-        for (int u = 0; u < 8; u++) acc = __fadd_rn(acc, fabsf(h2f(v[u])));
-    }
-    for (; j < out_dim; j++) acc = __fadd_rn(acc, fabsf(h2f(W[(size_t)j * in_dim + i])));
-    probes[i] = __half_as_ushort(__float2half_rn(__fdiv_rn(acc, (float)out_dim)));
+    return ((w & 0x7fffu) << 5) | ((uint32_t)(15 - p) << 1) | ((w >> 15) & 1u);
+}
+__device__ __forceinline__ uint16_t bucket_code(uint32_t key)
+{
+    return (uint16_t)(((key & 1u) << 15) | ((key >> 5) & 0x7ff0u) | (15u - ((key >> 1) & 15u)));
 }
 
-// sort within each bucket of 16: rank_p = #{q : |w_q| > |w_p|} + #{q < p : |w_q| == |w_p|}
-__global__ void k_bucket_sort(const uint16_t* __restrict__ W, int in_dim, int nb, uint16_t* __restrict__ buckets)
+// Batcher's odd-even merge sort of 16 keys, descending (63 comparators)
+__device__ __forceinline__ void sort16(uint32_t (&k)[16])
 {
-    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (size_t)in_dim * nb) return;
-    const int i = (int)(idx % in_dim);
-    const int b = (int)(idx / in_dim);
-    uint16_t v[16];
-    float key[16];
 #pragma unroll
-    for (int p = 0; p < 16; p++) v[p] = W[(size_t)(b * 16 + p) * in_dim + i];
+    for (int p = 1; p < 16; p *= 2)
 #pragma unroll
-    for (int p = 0; p < 16; p++) key[p] = fabsf(h2f(v[p]));
+        for (int q = p; q >= 1; q /= 2)
 #pragma unroll
-    for (int p = 0; p < 16; p++) {
-        int rank = 0;
+            for (int j = q % p; j <= 15 - q; j += 2 * q)
 #pragma unroll
-        for (int q = 0; q < 16; q++) rank += (key[q] > key[p]) || (key[q] == key[p] && q < p);
-        buckets[((size_t)i * 16 + rank) * nb + b] = (uint16_t)((v[p] & 0xFFF0u) | (unsigned)p);
-    }
+                for (int i = 0; i < q; i++)
+                    if (i + j + q < 16 && (i + j) / (p * 2) == (i + j + q) / (p * 2)) {
+                        const uint32_t a = k[i + j], b = k[i + j + q];
+                        k[i + j] = max(a, b);
+                        k[i + j + q] = min(a, b);
+                    }
 }
 
-// |original value| of row r = (i, rank) in bucket b: the position bits of the
-// packed code point back at W
-struct RowValues {
-    const uint16_t* W;
-    const uint16_t* brow;
-    int in_dim, i;
-    __device__ float operator()(int b) const
-    {
-        const int p = brow[b] & 15;
-        return fabsf(h2f(W[(size_t)(b * 16 + p) * in_dim + i]));
+// acc + |h|, h in the low or high half of w: one fp32 rounding, as the add's
+// (the product with 1 is exact)
+template <int HI>
+__device__ __forceinline__ float add_abs_half(float acc, uint32_t w)
+{
+    if constexpr (HI) asm("v_fma_mix_f32 %0, |%1|, 1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(acc) : "v"(w));
+    else asm("v_fma_mix_f32 %0, |%1|, 1.0, %0 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "+v"(acc) : "v"(w));
+    return acc;
+}
+
+// The block of numpy's pairwise summation (split at n/2 rounded down to a
+// multiple of 8 while n > 128) that holds element a of n: its end, and how
+// many subtrees end with it (each adds its left half's sum).
+__device__ __forceinline__ void pairwise_block(int n, int a, int& end, int& closes)
+{
+    int lo = 0;
+    closes = 0;
+    while (n > 128) {
+        int n2 = n / 2;
+        n2 -= n2 % 8;
+        if (a < lo + n2) {
+            n = n2;
+            closes = 0;
+        } else {
+            lo += n2;
+            n -= n2;
+            closes++;
+        }
     }
+    end = lo + n;
+}
+
+struct BucketLds {
+    uint32_t key[16 * kBkInputs * kBkKeyStride];            // [rank][column][bucket]
+    __align__(16) uint16_t raw[2][kBkInputs * kBkRawStride];   // [column][row of the chunk], two chunks
+    float tree[kBkDepth][16 * kBkInputs];                   // the pairwise sums waiting for their right halves
 };
 
-template <typename F>
-__device__ float pw_leaf(const F& f, int a, int n)
+// The block's work; WHOLE: it has all 16 columns (the last workgroup of an
+// in_dim that is no multiple of 16 re-reads its last one).
+template <bool WHOLE>
+__device__ __forceinline__ void bucketize_block(BucketLds& S, const uint16_t* __restrict__ W, int in_dim, int nb, int i0,
+                                                int ni, uint16_t* __restrict__ buckets, uint16_t* __restrict__ stats,
+                                                uint16_t* __restrict__ probes)
 {
-    if (n < 8) {
-        float res = -0.0f;
-        for (int i = 0; i < n; i++) res = __fadd_rn(res, f(a + i));
-        return res;
-    }
-    float r[8];
+#pragma clang fp contract(off)
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const bool worker = tid < kBkWorkers;
+    const int c2 = tid & 7, bl = tid >> 3;   // column pair and bucket of a sorting thread
+    const int ca = min(2 * c2, ni - 1), cb = min(2 * c2 + 1, ni - 1);
+    // columns 2*c2 and 2*c2 + 1 of a bucket's rows, as one 4-byte load at any
+    // 2-byte boundary; threads past the last bucket re-read it, so that every
+    // chunk has the same number of loads in flight
+    auto load = [&](int b0, uint32_t (&v)[16]) {
+        const uint16_t* p = W + (size_t)min(b0 + bl, nb - 1) * 16 * in_dim + i0;
 #pragma unroll
-    for (int j = 0; j < 8; j++) r[j] = f(a + j);
-    int i = 8;
-    for (; i < n - (n % 8); i += 8) {
-#pragma unroll
-        for (int j = 0; j < 8; j++) r[j] = __fadd_rn(r[j], f(a + i + j));
-    }
-    float res = __fadd_rn(__fadd_rn(__fadd_rn(r[0], r[1]), __fadd_rn(r[2], r[3])),
-                          __fadd_rn(__fadd_rn(r[4], r[5]), __fadd_rn(r[6], r[7])));
-    for (; i < n; i++) res = __fadd_rn(res, f(a + i));
-    return res;
-}
-
-// numpy's pairwise summation (blocks of <= 128, split at n/2 rounded down to
-// a multiple of 8), evaluated with an explicit stack
-template <typename F>
-__device__ float pairwise_sum(const F& f, int n)
-{
-    struct Frame {
-        int a, n, state;
-        float left;
+        for (int r = 0; r < 16; r++) {
+            typedef uint32_t u32u __attribute__((aligned(2)));
+            if constexpr (WHOLE) v[r] = *reinterpret_cast<const u32u*>(p + (size_t)r * in_dim + 2 * c2);
+            else v[r] = (uint32_t)p[(size_t)r * in_dim + ca] | ((uint32_t)p[(size_t)r * in_dim + cb] << 16);
+        }
     };
-    Frame st[24];
-    int sp = 0;
-    st[0] = {0, n, 0, 0.0f};
-    float result = 0.0f;
-    while (sp >= 0) {
-        Frame& fr = st[sp];
-        if (fr.n <= 128) {
-            result = pw_leaf(f, fr.a, fr.n);
-            sp--;
-            continue;
+    // the stats: wave w takes the rows (rank, column) 32w .. 32w + 31, eight
+    // at a time, lane = 8 * row + accumulator
+    constexpr int kRowSets = 16 * kBkInputs / (kBkWorkers / 8);
+    float acc[kRowSets];
+#pragma unroll
+    for (int s = 0; s < kRowSets; s++) acc[s] = 0.0f;
+    int depth = 0;      // pairwise sums on the stack (the same for every row)
+    int blk_end = 0, closes = 0;
+    // the ninth wave, lane = column: the column's sum over buckets g0 .. g1 - 1
+    // of a chunk; the next bucket's rows are read during this one's adds
+    float psum = 0.0f;
+    auto add_probes = [&](int buf, int g0, int g1) {
+        if (g0 >= g1) return;
+        const uint4* p = reinterpret_cast<const uint4*>(S.raw[buf] + (lane & 15) * kBkRawStride);
+        uint4 a = p[2 * g0], b = p[2 * g0 + 1];
+        for (int g = g0; g < g1; g++) {
+            const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            const int nx = min(g + 1, g1 - 1);
+            a = p[2 * nx];
+            b = p[2 * nx + 1];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                psum = add_abs_half<0>(psum, w[k]);
+                psum = add_abs_half<1>(psum, w[k]);
+            }
         }
-        int n2 = fr.n / 2;
-        n2 -= n2 % 8;
-        if (fr.state == 0) {
-            fr.state = 1;
-            st[sp + 1] = {fr.a, n2, 0, 0.0f};
-            sp++;
-        } else if (fr.state == 1) {
-            fr.left = result;
-            fr.state = 2;
-            st[sp + 1] = {fr.a + n2, fr.n - n2, 0, 0.0f};
-            sp++;
+    };
+    int nc_prev = 0;
+    auto chunk = [&](int b0, int buf, uint32_t (&v)[16]) {
+        const int nc = min(kBkChunk, nb - b0);
+        // ---- sort
+        if (worker) {
+            if (bl < nc) {
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const int c = 2 * c2 + h;
+                    uint32_t k[16], raw[8];
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        const uint32_t w = h ? v[r] >> 16 : v[r] & 0xffffu;
+                        k[r] = bucket_key(w, r);
+                        raw[r >> 1] = r & 1 ? raw[r >> 1] | (w << 16) : w;
+                    }
+                    uint4* rp = reinterpret_cast<uint4*>(S.raw[buf] + c * kBkRawStride + bl * 16);
+                    rp[0] = make_uint4(raw[0], raw[1], raw[2], raw[3]);
+                    rp[1] = make_uint4(raw[4], raw[5], raw[6], raw[7]);
+                    sort16(k);
+#pragma unroll
+                    for (int r = 0; r < 16; r++) S.key[(r * kBkInputs + c) * kBkKeyStride + bl] = k[r];
+                }
+            }
         } else {
-            result = __fadd_rn(fr.left, result);
-            sp--;
+            add_probes(buf ^ 1, nc_prev / 2, nc_prev);
+        }
+        nc_prev = nc;
+        __syncthreads();
+        // ---- emit: lane = 4 buckets (8 bytes at any 2-byte boundary) of one
+        // of 4 rows; then this buffer's next loads, behind the stores (the
+        // wait for them then waits for no later store)
+        if (worker) {
+            const int q = 4 * (lane & 15);
+#pragma unroll
+            for (int s = 0; s < 8; s++) {
+                const int rc = wave * 32 + s * 4 + (lane >> 4), r = rc / kBkInputs, c = rc % kBkInputs;
+                if (q >= nc || (!WHOLE && c >= ni)) continue;
+                const uint4 k = *reinterpret_cast<const uint4*>(S.key + rc * kBkKeyStride + q);
+                const uint32_t lo = bucket_code(k.x) | ((uint32_t)bucket_code(k.y) << 16);
+                const uint32_t hi = bucket_code(k.z) | ((uint32_t)bucket_code(k.w) << 16);
+                uint16_t* o = buckets + ((size_t)(i0 + c) * 16 + r) * nb + b0 + q;
+                typedef uint32_t u32x2u __attribute__((ext_vector_type(2), aligned(2)));
+                if (q + 4 <= nc) {
+                    *reinterpret_cast<u32x2u*>(o) = u32x2u{lo, hi};
+                } else {
+                    o[0] = (uint16_t)lo;
+                    if (q + 1 < nc) o[1] = (uint16_t)(lo >> 16);
+                    if (q + 2 < nc) o[2] = (uint16_t)hi;
+                }
+            }
+            load(b0 + 2 * kBkChunk, v);
+            const int row = wave * 32 + (lane >> 3), j = lane & 7;
+            for (int e = 0; e < nc;) {
+                if (b0 + e >= blk_end) pairwise_block(nb, b0 + e, blk_end, closes);
+                const int stop = min(nc, blk_end - b0);   // blocks start at multiples of 8
+                for (; e + 8 <= stop; e += 8) {
+#pragma unroll
+                    for (int s = 0; s < kRowSets; s++) {
+                        const uint32_t k = S.key[(row + 8 * s) * kBkKeyStride + e + j];
+                        acc[s] = __fadd_rn(acc[s], h2f((uint16_t)(k >> 5)));
+                    }
+                }
+                if (b0 + stop < blk_end) break;   // the block goes on in the next chunk
+                // the block's end: ((r0+r1) + (r2+r3)) + ((r4+r5) + (r6+r7)),
+                // the elements past its last whole 8 in order, then the
+                // subtrees it completes
+#pragma unroll
+                for (int s = 0; s < kRowSets; s++) {
+                    float a = acc[s];
+                    a = __fadd_rn(a, __shfl_down(a, 1, 8));
+                    a = __fadd_rn(a, __shfl_down(a, 2, 8));
+                    a = __fadd_rn(a, __shfl_down(a, 4, 8));
+                    acc[s] = 0.0f;
+                    if (j == 0) {
+                        for (int x = e; x < stop; x++)
+                            a = __fadd_rn(a, h2f((uint16_t)(S.key[(row + 8 * s) * kBkKeyStride + x] >> 5)));
+                        int d = depth;
+                        for (int x = 0; x < closes; x++) a = __fadd_rn(S.tree[--d][row + 8 * s], a);
+                        S.tree[d][row + 8 * s] = a;
+                    }
+                }
+                depth += 1 - closes;
+                e = stop;
+            }
+        } else {
+            add_probes(buf, 0, nc / 2);
+        }
+        __syncthreads();
+    };
+    uint32_t va[16], vb[16];
+    if (worker) {
+        load(0, va);
+        load(kBkChunk, vb);
+    } else {
+        __builtin_amdgcn_s_setprio(3);   // the serial chain goes first
+    }
+    int last = 0;   // the last chunk's buffer
+    for (int b0 = 0; b0 < nb; b0 += 2 * kBkChunk) {
+        chunk(b0, 0, va);
+        last = 0;
+        if (b0 + kBkChunk >= nb) break;
+        chunk(b0 + kBkChunk, 1, vb);
+        last = 1;
+    }
+    if (!worker) {
+        add_probes(last, nc_prev / 2, nc_prev);
+        if (lane < ni) probes[i0 + lane] = __half_as_ushort(__float2half_rn(__fdiv_rn(psum, (float)(nb * 16))));
+        return;
+    }
+    if (tid < 16 * kBkInputs) {   // row (rank, column) = tid: the tree's one remaining sum
+        const int r = tid / kBkInputs, c = tid % kBkInputs;
+        if (c < ni) {
+            const uint16_t m = __half_as_ushort(__float2half_rn(__fdiv_rn(__fadd_rn(0.0f, S.tree[0][tid]), (float)nb)));
+            const uint32_t m2 = (uint32_t)m | ((uint32_t)m << 16);
+            reinterpret_cast<uint2*>(stats)[(size_t)(i0 + c) * 16 + r] = make_uint2(m2, m2);
         }
     }
-    return result;
 }
 
-__global__ void k_bucket_stats(const uint16_t* __restrict__ W, const uint16_t* __restrict__ buckets, int in_dim,
-                               int nb, uint16_t* __restrict__ stats)
+__global__ __launch_bounds__(kBkThreads) void k_bucketize(const uint16_t* __restrict__ W, int in_dim, int nb,
+                                                          uint16_t* __restrict__ buckets,
+                                                          uint16_t* __restrict__ stats, uint16_t* __restrict__ probes)
 {
-    const size_t r = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= (size_t)in_dim * 16) return;
-    RowValues f{W, buckets + r * nb, in_dim, (int)(r / 16)};
-    const float s = __fadd_rn(0.0f, pairwise_sum(f, nb));
-    const uint16_t m = __half_as_ushort(__float2half_rn(__fdiv_rn(s, (float)nb)));
-    const uint32_t m2 = (uint32_t)m | ((uint32_t)m << 16);
-    reinterpret_cast<uint2*>(stats)[r] = make_uint2(m2, m2);
+    __shared__ BucketLds S;
+    const int i0 = xcd_remap((int)blockIdx.x, (int)gridDim.x) * kBkInputs;   // neighbours share W's lines in one L2
+    const int ni = min(kBkInputs, in_dim - i0);
+    if (ni == kBkInputs) bucketize_block<true>(S, W, in_dim, nb, i0, ni, buckets, stats, probes);
+    else bucketize_block<false>(S, W, in_dim, nb, i0, ni, buckets, stats, probes);
 }
 
 static unsigned grid_for(size_t n, unsigned block, unsigned cap = 65535u * 4)
@@ -217,15 +375,8 @@ int gen_f32(Ctx* c, uint64_t seed, uint64_t tid, size_t count, double mean, doub
 int bucketize(Ctx* c, const uint16_t* w, int out_dim, int in_dim, uint16_t* buckets, uint16_t* stats,
               uint16_t* probes)
 {
-    const int nb = out_dim / 16;
-    IAM_TRY(launch(c, "bucketize_probes", k_probes, dim3((in_dim + 255) / 256), dim3(256), 0, w, out_dim, in_dim,
-                   probes));
-    const size_t ncol = (size_t)in_dim * nb;
-    IAM_TRY(launch(c, "bucketize_sort", k_bucket_sort, dim3((unsigned)((ncol + 255) / 256)), dim3(256), 0, w,
-                   in_dim, nb, buckets));
-    const size_t rows = (size_t)in_dim * 16;
-    return launch(c, "bucketize_stats", k_bucket_stats, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, w,
-                  (const uint16_t*)buckets, in_dim, nb, stats);
+    return launch(c, "bucketize", k_bucketize, dim3((unsigned)((in_dim + kBkInputs - 1) / kBkInputs)), dim3(kBkThreads),
+                  0, w, in_dim, out_dim / 16, buckets, stats, probes);
 }
 
 }  // namespace iam

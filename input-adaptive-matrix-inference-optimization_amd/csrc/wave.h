@@ -2,12 +2,24 @@
 // 0x110 + n shifts within 16-lane rows, row_bcast15 / row_bcast31 = 0x142 /
 // 0x143 carry lane 15 / 31 of a row group into the next rows (masked by
 // row_mask).  Lanes with no source keep `old`.  The results are exact and
-// the order of operations is fixed, so they are deterministic.
+// the order of operations is fixed, so they are deterministic.  Also the
+// workgroup order that keeps neighbours on one XCD.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 namespace iam {
+
+// Blocks are dealt to the 8 XCDs round robin (block b -> XCD b % 8).  Remap
+// so that consecutive work items (the column tiles of one row slice, which
+// read the same stats, inputs and neighbouring lines of the same rows) land
+// on the same XCD and share its L2.
+__device__ __forceinline__ int xcd_remap(int b, int nblocks)
+{
+    const int q = nblocks >> 3, r = nblocks & 7;
+    const int xcd = b & 7, idx = b >> 3;
+    return xcd < r ? xcd * (q + 1) + idx : r * (q + 1) + (xcd - r) * q + idx;
+}
 
 template <int CTRL, int ROW_MASK = 0xF>
 __device__ __forceinline__ int dpp_i(int old, int v)

@@ -67,6 +67,24 @@ def test_gpu_bucketizer_matches_oracle(O, ctx, shape):
     assert np.array_equal(b, ob.ravel()) and np.array_equal(s, os_.ravel()) and np.array_equal(p, op)
 
 
+# one column, a ragged last workgroup, an odd row length, fewer than 8 buckets,
+# chunk and pairwise-block edges (64, 65, 128, 129, 136 and 1000 buckets)
+@pytest.mark.parametrize("shape", [(16, 1), (112, 17), (1024, 33), (1040, 16), (2048, 7), (2064, 48), (2176, 31),
+                                   (16000, 257)])
+def test_gpu_bucketizer_edges(O, ctx, shape):
+    """Byte equality with the oracle where the one-pass kernel's chunks, pairwise
+    blocks and column groups end, with ties, zeros of both signs and
+    infinities among the weights."""
+    W = O.gen_f16(5, 78, shape[0] * shape[1], 0.0, 0.02).reshape(shape).copy()
+    W[::7] = W[::7] & 0x8FFF          # subnormals and zeros
+    W[3::16, ::3] = W[2::16, ::3] ^ 0x8000   # equal magnitudes of opposite sign
+    W[5::64, ::5] = 0x7C00
+    W[6::64, ::5] = 0xFC00
+    b, s, p = _gpu_bucketize(ctx, W)
+    ob, os_, op = O.bucketize(W)
+    assert np.array_equal(b, ob.ravel()) and np.array_equal(s, os_.ravel()) and np.array_equal(p, op)
+
+
 def test_rmsnorm_and_add(O, ctx):
     x = O.gen_f32(0, 31, 4096, 0.0, 1.0)
     dlt = O.gen_f32(0, 32, 4096, 0.0, 0.5)
