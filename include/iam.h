@@ -372,9 +372,14 @@ int iam_model_forward(iam_model* m, int token, int pos, float effort, float* log
  * token_dev and pos is advanced, so a captured step replays without host
  * involvement.  hidden_override_dev, if non-NULL, replaces the embedding. */
 int iam_model_step_device(iam_model* m, float effort, const float* hidden_override_dev);
-/* Greedy decode (test_generation.cpp:197-276): feeds the prompt token by
- * token, then generates n_new tokens with first-max argmax.  With use_graph
- * the per-token step is captured once as a HIP graph and replayed.
+/* Greedy decode (test_generation.cpp:197-276): feeds the prompt, then
+ * generates n_new tokens with first-max argmax.  With use_graph the per-token
+ * step is captured once as a HIP graph and replayed.  The prompt's tokens
+ * before the last go through the model in batches where that is faster (fp64
+ * accumulation, from 8 to 16 tokens on by effort), in buffers the model keeps
+ * (about 2 MB a token, at most 512 tokens', at 4096 wide with FFN 14336); the
+ * KV cache, the picks in "history" and the walk counters are as by steps, and
+ * the last token's step leaves the activations and logits.
  * out_tokens receives n_new ids. */
 int iam_model_generate(iam_model* m, const int* prompt, int n_prompt, int n_new, float effort,
                        int use_graph, int* out_tokens);

@@ -36,6 +36,7 @@
 #include "accum.h"
 #include "internal.h"
 #include "layer_ops.h"
+#include "prefill.h"
 #include "search.h"
 #include "wave.h"
 
@@ -198,7 +199,7 @@ __device__ __forceinline__ float block_cutoff(const float* __restrict__ x, const
 // 4.9 us a launch against 6.4 with the radix search on 4 waves.
 constexpr int kCutWaves = 8;
 
-__global__ __launch_bounds__(64 * kCutWaves) void k_cutoff(CutoffArgs a)
+__device__ __forceinline__ float cutoff_block(const float* __restrict__ x, const uint16_t* __restrict__ probes, int quantile)
 {
     constexpr int VPT = kProbes / (64 * kCutWaves);
     union Scratch {
@@ -208,21 +209,48 @@ __global__ __launch_bounds__(64 * kCutWaves) void k_cutoff(CutoffArgs a)
     __shared__ __align__(16) uint4 s_scratch[(sizeof(Scratch) + 15) / 16];
     SearchLds<kCutWaves>& SL = *reinterpret_cast<SearchLds<kCutWaves>*>(s_scratch);
     WindowLds<kCutWaves>& WL = *reinterpret_cast<WindowLds<kCutWaves>*>(s_scratch);
-    const CutoffDesc& d = a.d[blockIdx.x];
     float xs[VPT], v[VPT];
     uint32_t pw[VPT / 2];
-    load_h16<VPT>(d.probes, pw);
-    load_f32<VPT>(d.x, xs);
+    load_h16<VPT>(probes, pw);
+    load_f32<VPT>(x, xs);
     window_clear<kCutWaves>(WL);
     importances<VPT>(xs, pw, v);
     __syncthreads();   // the histograms are clear
     float cut;
     bool hint_hit;
-    if (search_window<kCutWaves>(v, d.quantile, false, WL, cut, hint_hit, [](float) {}) != 1) {
+    if (search_window<kCutWaves>(v, quantile, false, WL, cut, hint_hit, [](float) {}) != 1) {
         __syncthreads();   // every wave is done with the window's scratch
-        cut = search_cutoff<kCutWaves>(v, d.quantile, SL);
+        cut = search_cutoff<kCutWaves>(v, quantile, SL);
     }
+    return cut;   // thread 0's
+}
+
+__global__ __launch_bounds__(64 * kCutWaves) void k_cutoff(CutoffArgs a)
+{
+    const CutoffDesc& d = a.d[blockIdx.x];
+    const float cut = cutoff_block(d.x, d.probes, d.quantile);
     if (threadIdx.x == 0) d.cutoff[0] = cut;
+}
+
+// The cutoffs of a prefill chunk: workgroup (token, matrix); the last token's
+// also go to the decode step's hints.
+struct TokenCutoffs {
+    const uint16_t* probes[kMaxMulti];
+    float* hints[kMaxMulti];
+    const float* x;   // [tokens][ld]
+    int ld;
+    int quantile;
+    float* cut;       // [n][kPfMaxTokens]
+};
+
+__global__ __launch_bounds__(64 * kCutWaves) void k_cutoff_tokens(TokenCutoffs a)
+{
+    const int t = blockIdx.x, m = blockIdx.y;
+    const float cut = cutoff_block(a.x + (size_t)t * a.ld, a.probes[m], a.quantile);
+    if (threadIdx.x == 0) {
+        a.cut[m * kPfMaxTokens + t] = cut;
+        if (t == (int)gridDim.x - 1 && a.hints[m]) *a.hints[m] = cut;
+    }
 }
 
 // ------------------------------------------------------------- dispatch ---
@@ -1377,6 +1405,21 @@ int bucketmul_dispatch(Ctx* c, int n, const MatOp* ops, int expert_no, float eff
     CutoffArgs args{};
     IAM_TRY(record_slots(c, n, ops, expert_no, effort, args));
     return launch(c, "bucket_cutoff", k_cutoff, dim3(n), dim3(64 * kCutWaves), 0, args);
+}
+
+int pf_cutoffs(Ctx* c, int n, const uint16_t* const* probes, const float* x, int ld, int tokens, int quantile, float* cut,
+               float* const* hints)
+{
+    TokenCutoffs a{};
+    for (int j = 0; j < n; j++) {
+        a.probes[j] = probes[j];
+        a.hints[j] = hints[j];
+    }
+    a.x = x;
+    a.ld = ld;
+    a.quantile = quantile;
+    a.cut = cut;
+    return launch(c, "prefill.cutoff", k_cutoff_tokens, dim3(tokens, n), dim3(64 * kCutWaves), 0, a);
 }
 
 // The selected-row list of slot i (k_dispatch), for the parity queries.

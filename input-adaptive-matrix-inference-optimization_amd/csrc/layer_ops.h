@@ -54,6 +54,10 @@ struct AttnLaunch {
     uint32_t* head_ctr = nullptr;      // [n_heads], zero on entry (left zero)
     void* zero_p = nullptr;
     int zero_n = 0;
+    // prefill: q and out hold n_batch tokens at positions pos0 .. (in place
+    // of *pos), each attending to the positions up to its own
+    int n_batch = 0;
+    int pos0 = 0;
 };
 int attention_launch(Ctx* c, const AttnLaunch& L);
 size_t attention_acc_words(int n_heads);

@@ -254,6 +254,9 @@ struct AttnArgs {
     int zero_n;
     int atomic_splits;       // model: runs per head group up to which o and l are added with atomics
     int kv_copies;           // qkv_acc: 2 when k and v have second copies after v (added here)
+    int n_batch;             // BATCH: the tokens of a prefill chunk, token n_batch - 1 - blockIdx.z at
+                             // position pos0 + token, its q and out a row of n_heads * 128 further
+    int pos0;
 };
 
 // LDS copies of the split's K and V rows: 128 fp16 + 8 of padding (68
@@ -263,7 +266,9 @@ struct AttnArgs {
 // bytes per lane of one V row (64 lanes, 64 banks).
 constexpr int kAttnRowStride = 128 + 8;
 
-template <typename Acc, int HPW>
+// BATCH: q and out of a prefill chunk's tokens, the longest contexts first,
+// one workgroup per head group and token (one run: its sums are the totals).
+template <typename Acc, int HPW, bool BATCH = false>
 __global__ __launch_bounds__(kAttnThreads) void k_attn(AttnArgs a, Acc scale)
 {
 #pragma clang fp contract(off)
@@ -285,12 +290,13 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn(AttnArgs a, Acc scale)
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int w = tid >> 6;
-    const int pos = *a.pos;
+    const int token = BATCH ? a.n_batch - 1 - (int)blockIdx.z : 0;
+    const int pos = BATCH ? a.pos0 + token : *a.pos;
     const int n_tok = min(pos + 1, a.max_ctx);
     // the context's chunks of 64 positions, dealt to at most kAttnGroups
     // workgroups per head group in runs of G consecutive chunks
     const int nch = (n_tok + kAttnChunk - 1) / kAttnChunk;
-    const int G = (nch + kAttnGroups - 1) / kAttnGroups;
+    const int G = BATCH ? nch : (nch + kAttnGroups - 1) / kAttnGroups;
     const int ng = (nch + G - 1) / G;       // workgroups of these heads with chunks
     const int grp = blockIdx.y;
     if (grp >= ng) return;                  // past the context: neither written nor counted
@@ -313,7 +319,7 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn(AttnArgs a, Acc scale)
             qv = hf == 0 ? __fsub_rn(__fmul_rn(lo, c), __fmul_rn(hi, sn))    // rope_mx: d < 64
                          : __fadd_rn(__fmul_rn(hi, c), __fmul_rn(lo, sn));   // d >= 64
         } else {
-            qv = a.q[(size_t)hq * HD + hf * DH + lane];
+            qv = a.q[((size_t)token * a.n_heads + hq) * HD + hf * DH + lane];
         }
         sq[w >> 1][hf * DH + lane] = (Acc)qv;
     }
@@ -465,6 +471,10 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn(AttnArgs a, Acc scale)
         if (tid < HPW * HD) atomicAdd(O + (size_t)(h0 + oj) * HD + od, (double)ot);
         if (tid >= HPW * HD && tid < HPW * HD + HPW)
             atomicAdd(O + (size_t)a.n_heads * HD + h0 + (tid - HPW * HD), sl[tid - HPW * HD]);
+        return;
+    }
+    if constexpr (BATCH) {
+        if (tid < HPW * HD) a.out[((size_t)token * a.n_heads + h0 + oj) * HD + od] = (float)((double)ot / sl[oj]);
         return;
     }
     // each head's sums of the run go to its own slot of the partials (no two
@@ -648,7 +658,7 @@ int attention_launch(Ctx* c, const AttnLaunch& L)
 {
     const int n_split = (L.max_ctx + kAttnChunk - 1) / kAttnChunk;
     IAM_REQUIRE(n_split <= kMaxAttnSplits, "attention: max_ctx above 8192");
-    IAM_REQUIRE(L.part && L.head_ctr && (L.out || L.acc), "attention: missing scratch");
+    IAM_REQUIRE(((L.part && L.head_ctr) || L.n_batch) && (L.out || L.acc), "attention: missing scratch");
     AttnArgs a{};
     a.q = L.q;
     a.qkv_acc = L.qkv_acc;
@@ -667,14 +677,22 @@ int attention_launch(Ctx* c, const AttnLaunch& L)
     a.zero_n = L.zero_n;
     a.atomic_splits = L.acc && !L.out ? L.atomic_splits : 0;
     a.kv_copies = L.kv_copies;
+    a.n_batch = L.n_batch;
+    a.pos0 = L.pos0;
     IAM_REQUIRE(L.n_heads <= kAttnMaxHeads, "attention: at most 512 query heads");
     // two query heads of one KV head per workgroup where the KV heads' query
     // heads pair up (each K and V value converted once for both): for 32
     // heads at most 32 runs x 16 workgroups, two resident per CU
     const bool pair = (L.n_heads / L.n_kv) % 2 == 0;
-    const dim3 grid(L.n_heads / (pair ? 2 : 1), attn_runs(L.max_ctx)), block(kAttnThreads);
+    const dim3 grid(L.n_heads / (pair ? 2 : 1), L.n_batch ? 1 : attn_runs(L.max_ctx), std::max(L.n_batch, 1)),
+        block(kAttnThreads);
     const double sd = 1.0 / std::sqrt(128.0);
     const float sf = 1.0f / std::sqrt(128.0f);
+    if (L.n_batch) {
+        IAM_REQUIRE(c->acc64 && L.out && !L.qkv_acc, "attention: a batch has fp64 sums, q and out");
+        return pair ? launch(c, "prefill.attention", k_attn<double, 2, true>, grid, block, 0, a, sd)
+                    : launch(c, "prefill.attention", k_attn<double, 1, true>, grid, block, 0, a, sd);
+    }
     if (c->acc64) return pair ? launch(c, "attention", k_attn<double, 2>, grid, block, 0, a, sd)
                               : launch(c, "attention", k_attn<double, 1>, grid, block, 0, a, sd);
     return pair ? launch(c, "attention", k_attn<float, 2>, grid, block, 0, a, sf)

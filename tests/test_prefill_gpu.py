@@ -1,0 +1,147 @@
+"""The batched prefill (generate's prompt tokens before the last) against the
+decode path token by token (forward), which the oracle tests pin.
+
+Both add the same exact fp64 products and round each output once; only the
+order of the additions differs, which can move an output across an fp32
+rounding boundary about once in 10^8 (2^-52 * a few roundings against 2^-24),
+and with it, once in 10^4 of those, a cached fp16 value.  So the caches are
+compared bit by bit with one part in 1000 allowed to differ by one fp16 ulp
+(a moved value travels through the layers after it), the picks with a tie's
+worth of room."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+BASE = dict(n_layers=2, dim=4096, ffn_dim=4096, n_heads=32, n_kv_heads=8, head_dim=128, vocab=512, max_ctx=128,
+            rope_theta=10000.0, norm_eps=1e-5)
+
+
+def make(iam, ctx, **kw):
+    m = iam.Model(ctx, iam.ModelConfig(**dict(BASE, **kw)))
+    m.synthesize(3)
+    return m
+
+
+def state(m, cfg, n):
+    kv = (cfg["n_layers"], cfg["max_ctx"], cfg["n_kv_heads"], 128)
+    k, v = (m.read_tensor(t, np.uint16).view(np.float16).reshape(kv)[:, :n] for t in ("kcache", "vcache"))
+    return k, v, m.read_tensor("history", np.int32)[1:n + 1], m.read_tensor("logits", np.float32)
+
+
+def ulp16(a, b):
+    """Distance in fp16 steps."""
+    def order(x):
+        i = x.view(np.int16).astype(np.int32)
+        return np.where(i < 0, -(i & 0x7FFF), i)
+    return np.abs(order(a) - order(b))
+
+
+def check(O, ctx, m, cfg, n, effort, seed=5):
+    prompt = O.gen_tokens(0, seed, n, cfg["vocab"])
+    m.reset_caches()
+    ctx.walk_counters(reset=True)
+    first = m.generate(prompt, 1, effort)
+    counted = ctx.walk_counters(reset=True)
+    k, v, hist, logits = state(m, cfg, n)
+    m.reset_caches()
+    log = ctx.empty(cfg["vocab"], np.float32)
+    picks = []
+    for pos, tok in enumerate(prompt):
+        m.forward(int(tok), pos, effort, log)
+        picks.append(O.argmax(log.read()))
+    wanted = ctx.walk_counters(reset=True)
+    wk, wv, _, _ = state(m, cfg, n)
+    want = log.read()
+    log.free()
+    for got, ref in ((k, wk), (v, wv)):
+        d = ulp16(got, ref)
+        assert np.mean(d != 0) < 1e-3 and d.max() <= 1, (n, effort, np.mean(d != 0), d.max())
+    assert np.mean(hist != np.array(picks)) <= 0.02
+    assert first[0] == hist[-1]
+    assert np.linalg.norm(logits - want) <= 1e-5 * np.linalg.norm(want)
+    # rows, bytes and matrices counted as the steps count them
+    assert counted[2] == wanted[2]
+    assert abs(counted[1] - wanted[1]) <= 1e-5 * wanted[1] and abs(counted[0] - wanted[0]) <= 1e-5 * wanted[0]
+
+
+@pytest.fixture(scope="module")
+def model(iam, ctx):
+    m = make(iam, ctx)
+    yield m
+    m.close()
+
+
+# too few tokens; one token group (part of one, all of it, and one or six
+# tokens more), two, three (the workgroups of four groups) and six groups,
+# whole and with a remainder the steps take or the batch takes
+@pytest.mark.parametrize("n,effort", [(5, 0.25), (16, 0.25), (10, 1.0), (17, 0.5), (18, 0.05), (23, 0.05), (33, 1.0),
+                                      (40, 0.25), (97, 0.125), (108, 0.25)])
+def test_token_groups(O, ctx, model, n, effort):
+    check(O, ctx, model, BASE, n, effort)
+
+
+@pytest.mark.parametrize("kw,n", [(dict(ffn_dim=4112, vocab=528), 40),                 # 257 and 33 bucket columns
+                                  (dict(dim=5120, n_heads=40, n_kv_heads=8, n_layers=1), 20),   # the norm apart
+                                  (dict(ffn_dim=5008, n_kv_heads=4, vocab=16, n_layers=1), 70)])
+def test_ragged_shapes(O, iam, ctx, kw, n):
+    cfg = dict(BASE, **kw)
+    m = make(iam, ctx, **kw)
+    try:
+        check(O, ctx, m, cfg, n, 0.25)
+    finally:
+        m.close()
+
+
+def test_weights_no_converter_writes(O, iam, ctx):
+    """Stats that rise with the rank (the selected ranks are not the first
+    ones), buckets with a position twice, and an embedding scale."""
+    m = make(iam, ctx)
+    try:
+        for name in ("layer0.wq", "layer1.w1", "layer1.w2"):
+            st = m.read_tensor(f"{name}.stats3", np.uint16).reshape(-1, 16)
+            st[::7] = st[::7, ::-1]
+            m.write_tensor(f"{name}.stats3", np.ascontiguousarray(st))
+        for name in ("layer0.wk", "layer0.w1", "lm_head"):
+            b = m.read_tensor(f"{name}.buckets", np.uint16)
+            b[::1009] = (b[::1009] & 0xFFF0) | 3
+            m.write_tensor(f"{name}.buckets", b)
+        m.set_embed_scale(np.linspace(0.5, 2.0, 4096).astype(np.float32))
+        check(O, ctx, m, BASE, 50, 0.25)
+    finally:
+        m.close()
+
+
+@pytest.mark.parametrize("block", [2, 16])
+def test_block_selection(O, ctx, model, block):
+    ctx.set_selection_block(block, 2.0)
+    try:
+        check(O, ctx, model, BASE, 20, 0.25)
+    finally:
+        ctx.set_selection_block(1, 2.0)
+
+
+def test_dense_head_and_continuation(O, iam, ctx, model):
+    """The dense LM head's picks, and tokens decoded after the prompt equal to
+    those after a prompt fed by steps."""
+    head = ctx.upload(O.gen_f16(0, 21, 512 * 4096, 0.0, 0.02))
+    prompt = O.gen_tokens(0, 6, 18, 512)
+    model.set_lm_dense(head)
+    try:
+        model.reset_caches()
+        got = model.generate(prompt, 6, 0.25)
+        hist = model.read_tensor("history", np.int32)[1:24]
+        model.reset_caches()
+        log = ctx.empty(512, np.float32)
+        seq = list(prompt)
+        for pos in range(23):
+            model.forward(int(seq[pos]), pos, 0.25, log)
+            pick = O.argmax(log.read())
+            assert hist[pos] == pick, pos
+            if pos >= 17:
+                seq.append(pick)
+        assert list(got) == seq[18:24]
+        log.free()
+    finally:
+        model.set_lm_dense(None)
+        head.free()
