@@ -547,11 +547,19 @@ __global__ __launch_bounds__(1024) void k_argmax(const float* __restrict__ v, in
     const int tid = threadIdx.x;
     float bv = -INFINITY;
     int bi = n;   // sentinel: larger than any index
-    for (int i = tid; i < n; i += 1024) {
-        const float x = v[i];
-        if (x > bv || (x == bv && i < bi)) {
-            bv = x;
-            bi = i;
+    // 16 loads in flight (one at a time: 12.6 us for 32000 values, the latency
+    // of 32 loads in a row; 16 or 32 at a time 7.4, one CU's misses); past the end the last value again, unused
+    for (int i0 = tid; i0 < n; i0 += 16 * 1024) {
+        float x[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++) x[u] = v[min(i0 + u * 1024, n - 1)];
+#pragma unroll
+        for (int u = 0; u < 16; u++) {
+            const int i = i0 + u * 1024;
+            if (i < n && (x[u] > bv || (x[u] == bv && i < bi))) {
+                bv = x[u];
+                bi = i;
+            }
         }
     }
     for (int o = 32; o > 0; o >>= 1) {

@@ -68,13 +68,16 @@ __global__ void k_rope_kv_rep32(const float* __restrict__ q, const float* __rest
 // the two (the tree's stride 64), and the strides 32 .. 1 follow as
 // shuffles, so the sum is the reference's work-group tree -- divided by
 // sqrt(128); e_t = exp(s_t) (no maximum subtracted) goes to e[h][t].  The
-// split's sum of e in position order goes to ssum[h][j].
+// split's sum of e in position order goes to ssum[h][j].  A wave holds its 16
+// K rows at once and runs their trees side by side: with a row loaded, summed
+// and finished before the next, the latencies added up (32 heads, 2047
+// positions: 13.8 -> 10.3 us, 33.5 MB).
 __global__ __launch_bounds__(256) void k_att32_score(const float* __restrict__ q, const float* __restrict__ kc,
                                                      const int* __restrict__ pos_p, int n_heads, int max_ctx,
                                                      float* __restrict__ e, float* __restrict__ ssum)
 {
 #pragma clang fp contract(off)
-    __shared__ float se[kSplit];
+    __shared__ __align__(16) float se[kSplit];
     const int h = blockIdx.x, j = blockIdx.y;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int n_tok = min(*pos_p + 1, max_ctx);
@@ -83,29 +86,68 @@ __global__ __launch_bounds__(256) void k_att32_score(const float* __restrict__ q
     if (nt <= 0) return;
     const float root = __fsqrt_rn((float)kHD);
     const float q0 = q[h * kHD + lane], q1 = q[h * kHD + 64 + lane];
-    for (int i = w; i < nt; i += 4) {
-        const float* kr = kc + ((size_t)(t0 + i) * n_heads + h) * kHD;
-        float a = __fadd_rn(__fmul_rn(q0, kr[lane]), __fmul_rn(q1, kr[64 + lane]));
+    // the wave's positions' K rows all loaded before the first is used (past
+    // the split: its last row again)
+    constexpr int PW = kSplit / 4;
+    float k0[PW], k1[PW];
 #pragma unroll
-        for (int st = 32; st > 0; st >>= 1) a = __fadd_rn(a, __shfl_down(a, st, 64));
-        if (lane == 0) {
-            const float ev = expf(__fdiv_rn(a, root));
-            se[i] = ev;
-            e[(size_t)h * max_ctx + t0 + i] = ev;
-        }
+    for (int u = 0; u < PW; u++) {
+        const float* kr = kc + ((size_t)(t0 + min(w + 4 * u, nt - 1)) * n_heads + h) * kHD;
+        k0[u] = kr[lane];
+        k1[u] = kr[64 + lane];
+    }
+    // the trees of all positions side by side; lane u then holds position u's
+    float a[PW], mine = 0.0f;
+#pragma unroll
+    for (int u = 0; u < PW; u++) a[u] = __fadd_rn(__fmul_rn(q0, k0[u]), __fmul_rn(q1, k1[u]));
+#pragma unroll
+    for (int st = 32; st > 0; st >>= 1)
+#pragma unroll
+        for (int u = 0; u < PW; u++) a[u] = __fadd_rn(a[u], __shfl_down(a[u], st, 64));
+#pragma unroll
+    for (int u = 0; u < PW; u++) {
+        const float v = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(a[u])));
+        if (lane == u) mine = v;
+    }
+    const int i = w + 4 * lane;
+    if (lane < PW) {
+        const float ev = i < nt ? expf(__fdiv_rn(mine, root)) : 0.0f;
+        se[i] = ev;
+        if (i < nt) e[(size_t)h * max_ctx + t0 + i] = ev;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        float s = 0.0f;
-        for (int i = 0; i < nt; i++) s = __fadd_rn(s, se[i]);
+        float4 v[kSplit / 4];
+#pragma unroll
+        for (int u = 0; u < kSplit / 4; u++) v[u] = *reinterpret_cast<const float4*>(se + 4 * u);
+        float s = 0.0f;   // past the split: + 0, which changes no sum of exponentials
+#pragma unroll
+        for (int u = 0; u < kSplit / 4; u++)
+            s = __fadd_rn(__fadd_rn(__fadd_rn(__fadd_rn(s, v[u].x), v[u].y), v[u].z), v[u].w);
         ssum[(size_t)h * gridDim.y + j] = s;
     }
+}
+
+// 0 + p[0] + p[step] + ..., in order, 16 loads in flight
+__device__ __forceinline__ float sum_in_order(const float* __restrict__ p, int step, int n)
+{
+    float s = 0.0f;
+    for (int i = 0; i < n; i += 16) {
+        float v[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++) v[u] = p[(size_t)min(i + u, n - 1) * step];
+#pragma unroll
+        for (int u = 0; u < 16; u++)
+            if (i + u < n) s = __fadd_rn(s, v[u]);
+    }
+    return s;
 }
 
 // Pass 2, workgroup (head h, split j), thread d: the total of the splits'
 // sums in split order, p_t = e_t / total (softmax_add32_mx), and the split's
 // sum of p_t * v_t[d] in position order (sumScores32's products) into
-// part[h][j][d].
+// part[h][j][d].  16 rows in flight, the first of them during the splits'
+// sums (10.9 -> 9.2 us).
 __global__ __launch_bounds__(kHD) void k_att32_pv(const float* __restrict__ vc, const int* __restrict__ pos_p,
                                                   int n_heads, int max_ctx, const float* __restrict__ e,
                                                   const float* __restrict__ ssum, float* __restrict__ part)
@@ -118,17 +160,38 @@ __global__ __launch_bounds__(kHD) void k_att32_pv(const float* __restrict__ vc, 
     const int nt = min(kSplit, n_tok - t0);
     if (nt <= 0) return;
     const int ns = (n_tok + kSplit - 1) / kSplit;
-    float total = 0.0f;
-    for (int s = 0; s < ns; s++) total = __fadd_rn(total, ssum[(size_t)h * gridDim.y + s]);
+    // the split's first V rows go out before the sums they wait for
+    const float* vr = vc + ((size_t)t0 * n_heads + h) * kHD + d;
+    const size_t step = (size_t)n_heads * kHD;
+    constexpr int B = 16;   // rows in flight
+    float v[B];
+#pragma unroll
+    for (int u = 0; u < B; u++) v[u] = vr[min(u, nt - 1) * step];
+    const float total = sum_in_order(ssum + (size_t)h * gridDim.y, 1, ns);
     if (d < nt) sp[d] = __fdiv_rn(e[(size_t)h * max_ctx + t0 + d], total);
     __syncthreads();
     float acc = 0.0f;
-    for (int i = 0; i < nt; i++)
-        acc = __fadd_rn(acc, __fmul_rn(sp[i], vc[((size_t)(t0 + i) * n_heads + h) * kHD + d]));
+    for (int i = 0; i < nt; i += B) {
+        float c[B];
+#pragma unroll
+        for (int u = 0; u < B; u++) {
+            c[u] = v[u];
+            v[u] = vr[min(i + B + u, nt - 1) * step];
+        }
+        if (i + B <= nt) {
+#pragma unroll
+            for (int u = 0; u < B; u++) acc = __fadd_rn(acc, __fmul_rn(sp[i + u], c[u]));
+        } else {
+#pragma unroll
+            for (int u = 0; u < B; u++)
+                if (i + u < nt) acc = __fadd_rn(acc, __fmul_rn(sp[i + u], c[u]));
+        }
+    }
     part[((size_t)h * gridDim.y + j) * kHD + d] = acc;
 }
 
-// Pass 3, workgroup h, thread d: out[h][d] = the splits' sums in split order.
+// Pass 3, workgroup h, thread d: out[h][d] = the splits' sums in split order
+// (9.1 us with a load at a time for 32 splits, 3.4 with 16 in flight).
 __global__ __launch_bounds__(kHD) void k_att32_sum(const int* __restrict__ pos_p, int max_ctx, int nsplit,
                                                    const float* __restrict__ part, float* __restrict__ out)
 {
@@ -136,9 +199,7 @@ __global__ __launch_bounds__(kHD) void k_att32_sum(const int* __restrict__ pos_p
     const int h = blockIdx.x, d = threadIdx.x;
     const int n_tok = min(*pos_p + 1, max_ctx);
     const int ns = n_tok > 0 ? (n_tok + kSplit - 1) / kSplit : 0;
-    float o = 0.0f;
-    for (int s = 0; s < ns; s++) o = __fadd_rn(o, part[((size_t)h * nsplit + s) * kHD + d]);
-    out[(size_t)h * kHD + d] = o;
+    out[(size_t)h * kHD + d] = sum_in_order(part + (size_t)h * nsplit * kHD + d, kHD, ns);
 }
 
 // ----------------------------------------------------------------- dense ---
@@ -148,7 +209,9 @@ __global__ __launch_bounds__(kHD) void k_att32_sum(const int* __restrict__ pos_p
 // wave holds a row's 256 work-items, lane i the four l = 4i .. 4i + 3 (one
 // 8-byte load per 256 columns); the tree's strides 128 .. 4 are shuffles
 // between lanes 32 .. 1 apart, strides 2 and 1 stay in lane 0.  x is staged
-// in LDS; each wave walks rows wave, wave + waves, ... two at a time.
+// in LDS; each wave walks rows wave, wave + waves, ... two at a time, eight
+// loads of a row in flight (32000 x 4096: 64.8 us with the loads the compiler
+// left between the adds, 46 with these, 5.7 TB/s).
 constexpr int kDenseThreads = 256;
 constexpr int kDenseMaxCols = 16384;
 
@@ -169,7 +232,26 @@ __global__ __launch_bounds__(kDenseThreads) void k_matmul16x32(const uint16_t* _
         const uint16_t* w = W + (size_t)r * cols;
 #pragma unroll
         for (int c = 0; c < 4; c++) s[c] = 0.0f;
-        for (int k = 0; k < nk; k++) {
+        int k = 0;
+        // whole columns blocks: 8 loads in flight a row, added in order
+        if constexpr (VEC) {
+            typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+            for (; (k + 8) * kDenseWG <= cols; k += 8) {
+                u32x2 p[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++)
+                    p[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(w + (k + u) * kDenseWG + 4 * lane));
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    const float4 xv = *reinterpret_cast<const float4*>(sx + (k + u) * kDenseWG + 4 * lane);
+                    s[0] = __fadd_rn(s[0], __fmul_rn(f16(p[u].x), xv.x));
+                    s[1] = __fadd_rn(s[1], __fmul_rn(f16(p[u].x >> 16), xv.y));
+                    s[2] = __fadd_rn(s[2], __fmul_rn(f16(p[u].y), xv.z));
+                    s[3] = __fadd_rn(s[3], __fmul_rn(f16(p[u].y >> 16), xv.w));
+                }
+            }
+        }
+        for (; k < nk; k++) {
             const int b = k * kDenseWG + 4 * lane;
             uint32_t v[4];
             if (VEC && b + 3 < cols) {

@@ -156,3 +156,25 @@ def test_model_dense_lm_head(iam, O, ctx, use_graph):
         dlm.free()
     finally:
         m.close()
+
+
+@pytest.mark.parametrize("rows,cols", [(9, 2048), (6, 2304), (3, 2044), (4, 3072)])
+def test_matmul_f16_dense_eight_blocks(O, ctx, rows, cols):
+    """Bit-exact where the eight-block loads end: exactly, with a block or
+    half of eight left, and just short of eight."""
+    test_matmul_f16_dense_bit_exact(O, ctx, rows, cols)
+
+
+@pytest.mark.parametrize("n", [1, 1023, 1025, 16384, 16385, 40001])
+def test_argmax_rounds(O, ctx, n):
+    """The first maximum at the ends of the threads' rounds of 16 values, with
+    the maximum repeated and the values past the end as large."""
+    v = O.gen_f32(3, n, n, 0.0, 1.0)
+    for at in ([0], [n - 1], [n // 2, n - 1]):
+        w = v.copy()
+        w[at] = 100.0
+        dv, di = ctx.upload(w), ctx.empty(1, np.int32)
+        ctx.argmax(dv, n, di)
+        assert di.read()[0] == at[0]
+        dv.free()
+        di.free()
