@@ -1315,7 +1315,20 @@ constexpr int kWalkWaves = 8;
 
 int sel_block_for(const Ctx* c, float effort) { return c->sel_block > 1 && effort < c->sel_below ? c->sel_block : 1; }
 
-void plan_walk(int n, const MatOp* ops, float effort, WalkPlan* plan, int blk, int tc)
+// A slice has rows for a full batch or two of every wave (128 rows each in
+// 64-column tiles) before the chip is filled: every slice adds into the same
+// outputs and, in the finalize modes, arrives at the same counters, one after
+// the other, so short slices cost more there than they save in the walk.  One
+// product at 1, 128, 192, 256, 320 and 512 rows a slice at least: 1024 x 4096
+// at effort 0.25 15.5, 12.0, 11.6, 11.4, 11.6 and 12.1 us, 2048 x 4096 14.6,
+// 14.1, 12.9, 11.7, 11.8 and 12.2, 4096 x 4096 at effort 0.05 13.4, 12.6, 11.9,
+// 11.5, 11.8 and 12.3.  With one to three columns a wave's load has few
+// lanes' worth of columns: 16 x 4096 12.4, 10.8 and (256) 12.1.  A decode step
+// without a finalize: 4 layers at effort 0.05 235.3 us at 1, 233.4 at 192, 235.9
+// at 256 (no change from effort 0.25 on, whose slices are longer).
+static double slice_rows(int cols, bool finalize) { return cols < 4 ? 128.0 : finalize ? 256.0 : 192.0; }
+
+void plan_walk(int n, const MatOp* ops, float effort, WalkPlan* plan, int blk, int tc, bool finalize)
 {
     double bytes[kMaxMulti], tot = 0;
     for (int i = 0; i < n; i++) {
@@ -1331,7 +1344,8 @@ void plan_walk(int n, const MatOp* ops, float effort, WalkPlan* plan, int blk, i
         WalkPlan& pl = plan[i];
         pl.NW = kWalkWaves;
         const double wgs = tot > 0 ? IAM_WALK_WGS * bytes[i] / tot : (double)IAM_WALK_WGS / n;
-        const int slices = std::max(1, (int)std::floor(wgs / pl.T + 1e-9));
+        const double full = est_rows(pl.n_in * 16, effort) / slice_rows(ops[i].mat.bucket_cols, finalize);
+        const int slices = std::max(1, (int)std::floor(std::min(wgs / pl.T + 1e-9, full)));
         pl.IPS = std::min(64 * pl.NW, std::max(1, (pl.n_in + slices - 1) / slices));
         if (blk > 1) pl.IPS = std::min(64 * pl.NW, (pl.IPS + blk - 1) / blk * blk);   // blocks within a slice
         pl.P = (pl.n_in + pl.IPS - 1) / pl.IPS;
@@ -1343,7 +1357,7 @@ int walk_tiles(int bucket_cols) { return (bucket_cols + kTileColsNarrow - 1) / k
 int max_slices(int n, const MatOp* ops, float effort, int blk, int tc)
 {
     WalkPlan plan[kMaxMulti];
-    plan_walk(n, ops, effort, plan, blk, tc);
+    plan_walk(n, ops, effort, plan, blk, tc, true);
     int P = 1;
     for (int i = 0; i < n; i++) P = std::max(P, plan[i].P);
     return P;
@@ -1497,7 +1511,7 @@ int walk_group(Ctx* c, const WalkGroup& g)
     const int blk = sel_block_for(c, g.effort);
     const int tc = walk_tile_cols(g);
     WalkPlan plan[kMaxMulti];
-    plan_walk(g.n, ops, g.effort, plan, blk, tc);
+    plan_walk(g.n, ops, g.effort, plan, blk, tc, g.fin != kFinNone);
     WalkArgs args{};
     args.sel_block = blk;
     args.n = g.n;

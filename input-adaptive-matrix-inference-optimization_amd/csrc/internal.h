@@ -218,8 +218,9 @@ struct WalkPlan {
     int P;      // slices
 };
 // blk: inputs per selection block (slices start at its multiples); tc:
-// columns per tile (the launch's walk_tile_cols)
-void plan_walk(int n, const MatOp* ops, float effort, WalkPlan* plan, int blk, int tc);
+// columns per tile (the launch's walk_tile_cols); finalize: the launch's tiles
+// are finished by their last workgroups (WalkFin)
+void plan_walk(int n, const MatOp* ops, float effort, WalkPlan* plan, int blk, int tc, bool finalize);
 // the selection block size of a walk at this effort
 int sel_block_for(const Ctx* c, float effort);
 
@@ -291,7 +292,7 @@ int walk_tile_cols(const WalkGroup& g);
 // column tiles of a matrix at the narrowest tile width (the most any launch
 // uses: the size of per-tile counters and candidates)
 int walk_tiles(int bucket_cols);
-// the largest slice count of the plan a walk of these matrices runs with
+// the largest slice count of the plan a finalizing walk of these matrices runs with
 // (selection blocks of blk inputs, tiles of tc columns)
 int max_slices(int n, const MatOp* ops, float effort, int blk, int tc);
 

@@ -379,6 +379,19 @@ def test_unaligned_rows_to_the_last(O, iam, ctx, out_dim, rows):
         assert S > 0.99 * rows
 
 
+@pytest.mark.parametrize("out_dim", [16, 48, 64, 1024])
+@pytest.mark.parametrize("effort", [0.0, 0.02, 0.3])
+def test_long_slices(O, iam, ctx, out_dim, effort):
+    """Narrow matrices and low efforts, whose slices are lengthened to hold
+    rows for the waves' batches: from 30 inputs a slice up to the 512 one
+    workgroup holds, in a full and in a partial last slice."""
+    b, s, p = make_matrix(O, out_dim, 4096, tid=8)
+    x = O.gen_f32(0, 10, 4096, 0.0, 1.0)
+    for kw in (dict(split=True), dict(split=False), dict(fused=iam)):
+        check_against_oracle(O, ctx, b, s, p, x, effort, **kw)
+    check_against_oracle(O, ctx, b[:4000 * 16], s[:4000 * 16], p, x, effort, in_size=4000, expert_rows=4000 * 16)
+
+
 def test_in_size_skips_rows(O, ctx):
     b, s, p = make_matrix(O, 256, 4096, tid=13)
     x = O.gen_f32(0, 14, 4096, 0.0, 1.0)
