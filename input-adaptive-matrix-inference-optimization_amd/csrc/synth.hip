@@ -88,11 +88,12 @@ __device__ __forceinline__ float h2f(uint16_t b) { return __half2float(__ushort_
 // 14336 x 4096, with the compact stats: 1420 us a call for three passes (the
 // probes with one load chain per column, a sort whose 2-byte stores lay 2 * nb
 // bytes apart, then the sums re-reading W through the codes' positions), now
-// 142 us; 2000 x 300: 32.9 -> 10.3 us.  W and the codes once at the part's
+// 138 us; 2000 x 300: 32.9 -> 10.3 us.  W and the codes once at the part's
 // copy rate are 47 us.  What bounds it now: the phases of the one workgroup a
 // CU holds follow each other (sorting, emitting and adding are about 50 us of
 // vector instructions, the waits between them as much again), and the probes'
-// chain of dependent adds takes issue slots from one SIMD (without it: 106 us).
+// chain of dependent adds takes issue slots from one SIMD (without it: 106 of
+// 142 us, measured before the emit's and the sums' LDS reads went out together).
 // 8 columns per workgroup, two to a CU: 226 us.
 constexpr int kBkInputs = 16;               // columns of W per workgroup
 constexpr int kBkChunk = 64;                // buckets per chunk
@@ -256,22 +257,35 @@ __device__ __forceinline__ void bucketize_block(BucketLds& S, const uint16_t* __
         // of 4 rows; then this buffer's next loads, behind the stores (the
         // wait for them then waits for no later store)
         if (worker) {
-            const int q = 4 * (lane & 15);
+            // (a full chunk's eight LDS reads go out together)
+            const int q = 4 * (lane & 15), rc0 = wave * 32 + (lane >> 4);
+            typedef uint32_t u32x2u __attribute__((ext_vector_type(2), aligned(2)));
+            auto codes = [](const uint4& k) -> u32x2u {
+                return u32x2u{bucket_code(k.x) | ((uint32_t)bucket_code(k.y) << 16),
+                              bucket_code(k.z) | ((uint32_t)bucket_code(k.w) << 16)};
+            };
+            auto row_out = [&](int rc) {
+                return buckets + ((size_t)(i0 + rc % kBkInputs) * 16 + rc / kBkInputs) * nb + b0 + q;
+            };
+            if (WHOLE && nc == kBkChunk) {
+                uint4 k[8];
 #pragma unroll
-            for (int s = 0; s < 8; s++) {
-                const int rc = wave * 32 + s * 4 + (lane >> 4), r = rc / kBkInputs, c = rc % kBkInputs;
-                if (q >= nc || (!WHOLE && c >= ni)) continue;
-                const uint4 k = *reinterpret_cast<const uint4*>(S.key + rc * kBkKeyStride + q);
-                const uint32_t lo = bucket_code(k.x) | ((uint32_t)bucket_code(k.y) << 16);
-                const uint32_t hi = bucket_code(k.z) | ((uint32_t)bucket_code(k.w) << 16);
-                uint16_t* o = buckets + ((size_t)(i0 + c) * 16 + r) * nb + b0 + q;
-                typedef uint32_t u32x2u __attribute__((ext_vector_type(2), aligned(2)));
-                if (q + 4 <= nc) {
-                    *reinterpret_cast<u32x2u*>(o) = u32x2u{lo, hi};
-                } else {
-                    o[0] = (uint16_t)lo;
-                    if (q + 1 < nc) o[1] = (uint16_t)(lo >> 16);
-                    if (q + 2 < nc) o[2] = (uint16_t)hi;
+                for (int s = 0; s < 8; s++) k[s] = *reinterpret_cast<const uint4*>(S.key + (rc0 + 4 * s) * kBkKeyStride + q);
+#pragma unroll
+                for (int s = 0; s < 8; s++) *reinterpret_cast<u32x2u*>(row_out(rc0 + 4 * s)) = codes(k[s]);
+            } else {
+                for (int s = 0; s < 8; s++) {
+                    const int rc = rc0 + 4 * s;
+                    if (q >= nc || rc % kBkInputs >= ni) continue;
+                    const u32x2u c = codes(*reinterpret_cast<const uint4*>(S.key + rc * kBkKeyStride + q));
+                    uint16_t* o = row_out(rc);
+                    if (q + 4 <= nc) {
+                        *reinterpret_cast<u32x2u*>(o) = c;
+                    } else {
+                        o[0] = (uint16_t)c.x;
+                        if (q + 1 < nc) o[1] = (uint16_t)(c.x >> 16);
+                        if (q + 2 < nc) o[2] = (uint16_t)c.y;
+                    }
                 }
             }
             load(b0 + 2 * kBkChunk, v);
@@ -279,6 +293,17 @@ __device__ __forceinline__ void bucketize_block(BucketLds& S, const uint16_t* __
             for (int e = 0; e < nc;) {
                 if (b0 + e >= blk_end) pairwise_block(nb, b0 + e, blk_end, closes);
                 const int stop = min(nc, blk_end - b0);   // blocks start at multiples of 8
+                for (; e + 32 <= stop; e += 32) {   // 16 LDS reads in flight
+                    uint32_t k[4][kRowSets];
+#pragma unroll
+                    for (int u = 0; u < 4; u++)
+#pragma unroll
+                        for (int s = 0; s < kRowSets; s++) k[u][s] = S.key[(row + 8 * s) * kBkKeyStride + e + 8 * u + j];
+#pragma unroll
+                    for (int u = 0; u < 4; u++)
+#pragma unroll
+                        for (int s = 0; s < kRowSets; s++) acc[s] = __fadd_rn(acc[s], h2f((uint16_t)(k[u][s] >> 5)));
+                }
                 for (; e + 8 <= stop; e += 8) {
 #pragma unroll
                     for (int s = 0; s < kRowSets; s++) {
