@@ -4,7 +4,7 @@
 Workload: 32 layers, dim 4096, FFN 14336, 32 query / 8 KV heads of 128,
 vocabulary 32000 with a bucket-layout LM head, fp16 GQA KV cache of 4096
 positions, RoPE theta 10000; random-init synthetic weights N(0, 0.02^2)
-bucketized on the GPU; a 512-token random-id prompt fed token by token; then
+bucketized on the GPU; a 512-token random-id prompt fed; then
 greedy decode at effort 0.25.  A step is one decode token (captured once as a
 HIP graph and replayed).  `value` is decode tokens per second, timed with
 the library's walk counting switched off; the bytes per token come from

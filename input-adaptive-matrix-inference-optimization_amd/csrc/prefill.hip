@@ -201,6 +201,10 @@ __device__ __forceinline__ void fma_below(double& acc, double w, uint32_t rank, 
                  : "vcc");
 }
 
+// A vector instruction's write of exec wants 4 wait states before a lane read
+// or write; the compiler, which spills scalars with those, sees none in the asm
+__device__ __forceinline__ void exec_settled() { asm volatile("s_nop 3"); }
+
 template <int WT>
 __global__ __launch_bounds__(256, 3) void k_pf_products(PfGemmArgs a)
 {
@@ -271,6 +275,7 @@ __global__ __launch_bounds__(256, 3) void k_pf_products(PfGemmArgs a)
                 for (int o = 0; o < OPL; o++)
                     fma_below(acc[t][o], w, out == (uint32_t)o ? 0u : 1u, xd[(size_t)i * kPfGroup + t], 1u);
             }
+            exec_settled();
         }
     };
     // An input's scalar loads (its tokens' x and counts), issued one input
@@ -316,6 +321,7 @@ __global__ __launch_bounds__(256, 3) void k_pf_products(PfGemmArgs a)
 #pragma unroll
             for (int o = 0; o < OPL; o++) fma_below(acc[t][o], w[o], rank[o], x[t], nt);
         }
+        exec_settled();
     };
     for (int k = k0; k < k1; k += kPfInputs, buf ^= 1, turn = turn == 2 ? 0 : turn + 1) {
         uint32_t perm0 = 0, perm1 = 0;
