@@ -492,7 +492,8 @@ static size_t pf_layout(const iam_model* m, int tokens, char* base, PfBuffers* B
         at += (bytes + 255) / 256 * 256;
         return p;
     };
-    // the widest partial sums of the step
+    // the widest partial sums of the step (the LM head's too where the dense
+    // one is set: the buffers outlive that choice)
     auto part = [&](int n, const Mat* const* w, size_t width) {
         iam_bucket_matrix mats[kMaxMulti];
         for (int j = 0; j < n; j++) mats[j] = w[j]->desc();
@@ -502,7 +503,7 @@ static size_t pf_layout(const iam_model* m, int tokens, char* base, PfBuffers* B
     const Mat *qkv[] = {&ly.wq, &ly.wk, &ly.wv}, *o[] = {&ly.wo}, *up[] = {&ly.w1, &ly.w3}, *down[] = {&ly.w2},
               *lm[] = {&m->lm};
     const size_t p = std::max({part(3, qkv, D + 2 * KVD), part(1, o, D), part(2, up, 2 * F), part(1, down, D),
-                               m->lm_dense ? (size_t)0 : part(1, lm, C.vocab)});
+                               part(1, lm, C.vocab)});
     PfBuffers b{};
     b.h = (float*)take(M * D * 4);
     b.x = (float*)take(M * K * 4);

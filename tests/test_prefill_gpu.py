@@ -145,3 +145,21 @@ def test_dense_head_and_continuation(O, iam, ctx, model):
     finally:
         model.set_lm_dense(None)
         head.free()
+
+
+def test_buffers_hold_the_bucket_head_after_the_dense_one(O, iam, ctx):
+    """The prefill buffers, first allocated under the dense head, hold the
+    bucket-layout head's partial sums, the widest here, afterwards."""
+    cfg = dict(BASE, n_layers=1, vocab=32000)
+    m = make(iam, ctx, n_layers=1, vocab=32000)
+    head = ctx.upload(O.gen_f16(0, 22, 32000 * 4096, 0.0, 0.02))
+    try:
+        m.set_lm_dense(head)
+        m.generate(O.gen_tokens(0, 7, 100, 32000), 1, 0.25)
+        m.set_lm_dense(None)
+        before = ctx.mem_status()[0]
+        check(O, ctx, m, cfg, 100, 0.25)
+        assert ctx.mem_status()[0] == before
+    finally:
+        m.close()
+        head.free()
