@@ -1674,7 +1674,14 @@ static int bucketmul_whole(Ctx* c, int n, const MatOp* ops, int expert_no, float
 {
     CutoffArgs args{};
     IAM_TRY(record_slots(c, n, ops, expert_no, effort, args));
-    return walk_slots(c, n, ops, kInX, nullptr, nullptr, 0.0f, false);
+    const int rc = walk_slots(c, n, ops, kInX, nullptr, nullptr, 0.0f, false);
+    if (rc == IAM_OK) return rc;
+    // Refused (an output, the buckets, no room for the scratch): the dispatch
+    // that was recorded stands all the same, for a mul or a query after it, so
+    // its cutoffs are found by the search launch.
+    const std::string why = iam_last_error();
+    (void)launch(c, "bucket_cutoff", k_cutoff, dim3(n), dim3(64 * kCutWaves), 0, args);
+    return fail(rc, why);
 }
 
 // One matrix group in one launch: every workgroup computes the input (x, or

@@ -454,6 +454,33 @@ def test_multi_matches_single(iam, O, ctx):
         d.free()
 
 
+@pytest.mark.parametrize("call", ["full", "multi"])
+def test_dispatch_of_a_refused_product(O, iam, ctx, call):
+    """A full or multi call refused for its outputs leaves its dispatch: the
+    queries and a mul after it use that one's cutoff, not an earlier call's."""
+    b, s, p = make_matrix(O, 1024, 4096, tid=5)
+    x = O.gen_f32(0, 3, 4096, 0.0, 1.0)
+    check_against_oracle(O, ctx, b, s, p, 4.0 * x, 0.5)   # another cutoff in the slot
+    oy, ocut, omask, oS = O.bucketmul(x, s, p, b, 0.125)
+    bufs = [ctx.upload(a) for a in (b, s, p, x)] + [ctx.empty(1024 + 4, np.float32)]
+    db, ds, dp, dx, dy = bufs
+    try:
+        with pytest.raises(iam.IamError):
+            if call == "full":
+                ctx.full_mul(dx, ds, dp, db, 0, 4096, 64, 65536, 0.125, dy.ptr + 4)
+            else:
+                ctx.multi([iam.BucketMatrix(db.ptr, ds.ptr, dp.ptr, 65536, 64, 4, 3)], [dx], [4096], [dy.ptr + 4], 0.125)
+        ctx.mul(db, 64, dy)
+        y = dy.read(np.float32, 1024)
+        cut, S = ctx.dispatch_info(0)
+        assert np.float32(cut).view(np.uint32) == np.float32(ocut).view(np.uint32)
+        assert S == oS == ctx.walk_count(0)
+        assert rel_l2(y, oy) <= RTOL_L2
+    finally:
+        for d in bufs:
+            d.free()
+
+
 def test_invalid_arguments_raise(iam, O, ctx):
     b, s, p = make_matrix(O, 64, 4096, tid=25)
     db, ds, dp = ctx.upload(b), ctx.upload(s), ctx.upload(p)
