@@ -53,7 +53,9 @@ const char* iam_last_error(void);
 /* device name / CU count / global memory (gpu.hpp:123-135, :28-31) */
 int iam_device_info(iam_ctx* ctx, char* name, size_t name_len, int* compute_units,
                     size_t* global_mem_bytes);
-/* MemoryTracker (gpu.hpp:21-60): byte budget = device memory - margin. */
+/* MemoryTracker (gpu.hpp:21-60): byte budget = device memory - margin.
+ * allocated counts the prefill buffers the models keep (iam_model_generate);
+ * an allocation that finds no room frees those first. */
 int iam_mem_status(iam_ctx* ctx, size_t* allocated, size_t* usable);
 
 /* Gpu::createBuffer (gpu.hpp:236-262) */
@@ -377,7 +379,8 @@ int iam_model_step_device(iam_model* m, float effort, const float* hidden_overri
  * step is captured once as a HIP graph and replayed.  The prompt's tokens
  * before the last go through the model in batches where that is faster (fp64
  * accumulation, from 8 to 16 tokens on by effort), in buffers the model keeps
- * (about 2 MB a token, at most 512 tokens', at 4096 wide with FFN 14336); the
+ * until an allocation needs their room (about 2 MB a token, at most 512
+ * tokens', at 4096 wide with FFN 14336; fewer where there is less room); the
  * KV cache, the picks in "history" and the walk counters are as by steps, and
  * the last token's step leaves the activations and logits.
  * out_tokens receives n_new ids. */

@@ -88,6 +88,13 @@ struct PendingEvent {
     hipEvent_t start, stop;
 };
 
+// A buffer that its owner makes again when it needs it and finds it gone
+// (a model's prefill buffers): nothing in it outlives the owner's call.
+struct Spare {
+    char* p = nullptr;
+    int cap = 0;   // what p holds, in the owner's units (0: nothing)
+};
+
 struct Ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -95,6 +102,7 @@ struct Ctx {
     size_t usable = 0;
     size_t allocated = 0;
     std::map<uintptr_t, size_t> allocs;   // base -> bytes
+    std::vector<Spare*> spares;           // freed when an allocation finds no room
     bool profiling = false;
     bool capturing = false;
     std::vector<PendingEvent> pending;
@@ -138,6 +146,7 @@ int ctx_alloc(Ctx* c, size_t bytes, void** out);
 // IAM_OK if [p, p+bytes) lies inside one allocation of this context
 int check_dev_range(Ctx* c, const void* p, size_t bytes, const char* what);
 int ctx_free(Ctx* c, void* p);
+int spare_free(Ctx* c, Spare& s);
 int ensure_slot(Ctx* c, int slot);
 int ensure_list(Ctx* c, int slot, int chunks);
 // the walk scratch of a slot: accumulators for m outputs, T tile counters,

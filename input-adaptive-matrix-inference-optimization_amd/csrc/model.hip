@@ -21,6 +21,7 @@
 // prompt's tokens before the last go through the layers in batches (prefill.hip).
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -106,10 +107,10 @@ struct iam_model {
     // decode loops launch the latter while that many remain, so the gap
     // between two graph launches comes once per kGraphSteps steps)
     iam::StepGraph one, multi;
-    // the batched prefill's buffers, for chunks of up to pf_cap tokens
-    // (0: none; grown by prefill, at most kPfMaxTokens)
-    char* pf_mem = nullptr;
-    int pf_cap = 0;
+    // the batched prefill's buffers, for chunks of up to pf.cap tokens (grown
+    // by prefill, at most kPfMaxTokens; given back where the context's memory
+    // is wanted for something else)
+    iam::Spare pf;
     std::vector<void*> owned;
 };
 
@@ -473,7 +474,7 @@ static int pf_take(int tokens, float effort)
     return rest >= 6.0 / scale ? tokens : whole;
 }
 
-// The buffers of one prefill chunk, laid out in pf_mem.
+// The buffers of one prefill chunk, laid out in pf.p.
 struct PfBuffers {
     float *h, *x, *q, *cut;
     double *xd, *part;
@@ -520,23 +521,24 @@ static size_t pf_layout(const iam_model* m, int tokens, char* base, PfBuffers* B
     return at;
 }
 
-// Buffers for chunks of `tokens`, or false: no memory for them.
+// Buffers for chunks of `tokens`, or of as many as there is room for (half as
+// many groups at a time, what there was before among them); false: none.
 static bool pf_ensure(iam_model* m, int tokens)
 {
-    if (tokens <= m->pf_cap) return true;
+    if (tokens <= m->pf.cap) return true;
     Ctx* c = m->c;
-    if (m->pf_mem && ctx_free(c, m->pf_mem) != IAM_OK) return false;
-    m->pf_mem = nullptr;
-    m->pf_cap = 0;
-    // a chunk of fewer tokens may split its products further: the largest of all
-    size_t bytes = 0;
-    for (int g = 1; g <= pf_groups(tokens); g++) bytes = std::max(bytes, pf_layout(m, g * kPfGroup, nullptr, nullptr));
-    if (ctx_alloc(c, bytes, (void**)&m->pf_mem) != IAM_OK) {
-        m->pf_mem = nullptr;
-        return false;
+    const int had = m->pf.cap / kPfGroup;
+    if (m->pf.p && spare_free(c, m->pf) != IAM_OK) return false;
+    for (int G = pf_groups(tokens); G >= 1; G = G > had ? std::max(G / 2, had) : G / 2) {
+        // a chunk of fewer tokens may split its products further: the largest of all
+        size_t bytes = 0;
+        for (int g = 1; g <= G; g++) bytes = std::max(bytes, pf_layout(m, g * kPfGroup, nullptr, nullptr));
+        if (ctx_alloc(c, bytes, (void**)&m->pf.p) == IAM_OK) {
+            m->pf.cap = G * kPfGroup;
+            return true;
+        }
     }
-    m->pf_cap = pf_groups(tokens) * kPfGroup;
-    return true;
+    return false;
 }
 
 // One product group of the chunk: cutoffs, selection, products of x.
@@ -623,11 +625,12 @@ static int prefill_batched(iam_model* m, const int* prompt, int n, float effort,
     *done = 0;
     const int largest = pf_take(std::min(n, kPfMaxTokens), effort);
     if (largest == 0 || !m->c->acc64 || !pf_ensure(m, largest)) return IAM_OK;
+    const int most = std::min(kPfMaxTokens, m->pf.cap);
     while (*done < n) {
-        const int chunk = std::min(n - *done, kPfMaxTokens), tokens = pf_take(chunk, effort);
+        const int chunk = std::min(n - *done, most), tokens = pf_take(chunk, effort);
         if (tokens == 0) break;
         PfBuffers B;
-        (void)pf_layout(m, tokens, m->pf_mem, &B);
+        (void)pf_layout(m, tokens, m->pf.p, &B);
         IAM_TRY(iam_write(static_cast<iam_ctx*>(m->c), B.tokens, 0, prompt + *done, (size_t)tokens * 4));
         IAM_TRY(pf_chunk(m, B, *done, tokens, effort));
         *done += tokens;
@@ -754,6 +757,7 @@ int iam_model_create(iam_ctx* c, const iam_model_config* cfg, iam_model** out)
     m->c = c;
     m->cfg = C;
     m->layers.resize(C.n_layers);
+    c->spares.push_back(&m->pf);
     const int D = C.dim, F = C.ffn_dim, KVD = C.n_kv_heads * C.head_dim;
     int rc = IAM_OK;
     auto T = [&](int r) {
@@ -823,7 +827,9 @@ int iam_model_destroy(iam_model* m)
     if (!m) return IAM_OK;
     (void)hipStreamSynchronize(m->c->stream);
     drop_graph(m);
-    if (m->pf_mem) (void)ctx_free(m->c, m->pf_mem);
+    auto& spares = m->c->spares;
+    spares.erase(std::remove(spares.begin(), spares.end(), &m->pf), spares.end());
+    if (m->pf.p) (void)spare_free(m->c, m->pf);
     for (void* p : m->owned) (void)ctx_free(m->c, p);
     delete m;
     return IAM_OK;

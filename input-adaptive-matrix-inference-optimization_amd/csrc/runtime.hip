@@ -20,12 +20,29 @@ int fail(int code, const std::string& msg)
     return code;
 }
 
+// hipFree waits for the work that may still use the buffer
+int spare_free(Ctx* c, Spare& s)
+{
+    IAM_TRY(ctx_free(c, s.p));
+    s = Spare{};
+    return IAM_OK;
+}
+
+// Frees every spare buffer; whether there was one.
+static bool free_spares(Ctx* c)
+{
+    bool any = false;
+    for (Spare* s : c->spares) any |= s->p && spare_free(c, *s) == IAM_OK;
+    return any;
+}
+
 int ctx_alloc(Ctx* c, size_t bytes, void** out)
 {
     if (!out) return fail(IAM_E_INVALID, "alloc: null output pointer");
     *out = nullptr;
     if (bytes == 0) bytes = 1;
     // MemoryTracker::can_allocate (gpu.hpp:40-44)
+    if (c->allocated + bytes > c->usable) free_spares(c);
     if (c->allocated + bytes > c->usable)
         return fail(IAM_E_NOMEM, "alloc: over the context's device memory budget (budget " +
                                      std::to_string(c->usable) + " bytes, in use " +
@@ -35,6 +52,12 @@ int ctx_alloc(Ctx* c, size_t bytes, void** out)
     hipError_t e = hipMalloc(&p, bytes);
     if (e != hipSuccess) {
         (void)hipGetLastError();
+        if (free_spares(c)) {
+            e = hipMalloc(&p, bytes);
+            if (e != hipSuccess) (void)hipGetLastError();
+        }
+    }
+    if (e != hipSuccess) {
         return fail(IAM_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     }
     c->allocs[(uintptr_t)p] = bytes;

@@ -8,6 +8,8 @@ and with it, once in 10^4 of those, a cached fp16 value.  So the caches are
 compared bit by bit with one part in 1000 allowed to differ by one fp16 ulp
 (a moved value travels through the layers after it), the picks with a tie's
 worth of room."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -37,11 +39,14 @@ def ulp16(a, b):
     return np.abs(order(a) - order(b))
 
 
-def check(O, ctx, m, cfg, n, effort, seed=5):
+def check(O, ctx, m, cfg, n, effort, seed=5, after=None):
+    """after: called once the prompt has been fed."""
     prompt = O.gen_tokens(0, seed, n, cfg["vocab"])
     m.reset_caches()
     ctx.walk_counters(reset=True)
     first = m.generate(prompt, 1, effort)
+    if after:
+        after()
     counted = ctx.walk_counters(reset=True)
     k, v, hist, logits = state(m, cfg, n)
     m.reset_caches()
@@ -163,3 +168,72 @@ def test_buffers_hold_the_bucket_head_after_the_dense_one(O, iam, ctx):
     finally:
         m.close()
         head.free()
+
+
+class Budget:
+    """The context's memory budget set to a number of bytes.  There is no call
+    for that: the field (after the device, the stream and the total) is written
+    in place, and mem_status has to read it back."""
+
+    def __init__(self, ctx):
+        self.ctx = ctx
+        self.field = ctypes.c_size_t.from_address(ctx.h.value + 24)
+        self.usable = ctx.mem_status()[1]
+        assert self.field.value == self.usable
+
+    def set(self, n):
+        self.field.value = n
+        assert self.ctx.mem_status()[1] == n
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *a):
+        self.set(self.usable)
+
+
+def test_prefill_buffers_make_room(O, iam):
+    """What a context without prefill buffers can allocate, it can allocate
+    with them too (they are freed), and a prompt after that is as before."""
+    with iam.Ctx(0) as ctx, Budget(ctx) as budget:
+        m = make(iam, ctx, n_layers=1)
+        bare = ctx.mem_status()[0]
+        check(O, ctx, m, dict(BASE, n_layers=1), 60, 0.25)
+        kept = ctx.mem_status()[0]
+        assert kept > bare
+        budget.set(kept + 4096)
+        buf = ctx.alloc(kept - bare)
+        assert ctx.mem_status()[0] == kept
+        # no room now: by steps
+        check(O, ctx, m, dict(BASE, n_layers=1), 60, 0.25)
+        assert ctx.mem_status()[0] == kept
+        buf.free()
+        check(O, ctx, m, dict(BASE, n_layers=1), 60, 0.25)
+        assert ctx.mem_status()[0] == kept
+        m.close()
+        assert ctx.mem_status()[0] < kept
+
+
+@pytest.mark.parametrize("n", [65, 97])
+def test_prefill_in_chunks_that_fit(O, iam, n):
+    """Where the buffers of the whole prompt find no room, the prompt goes in
+    smaller batches, and smaller buffers that are there already stay in use."""
+    cfg = dict(BASE, n_layers=1)
+    with iam.Ctx(0) as ctx, Budget(ctx) as budget:
+        m = make(iam, ctx, n_layers=1)
+        check(O, ctx, m, cfg, 33, 0.25)                     # buffers of two groups
+        two = ctx.mem_status()[0]
+        names = []
+
+        def batched():
+            ctx.profiling(False)
+            names.append(ctx.kernel_stat("prefill.products")[1])
+
+        budget.set(two + 4096)
+        ctx.kernel_stats_reset()
+        ctx.profiling(True)
+        check(O, ctx, m, cfg, n, 0.25, after=lambda: (ctx.sync(), batched()))
+        assert ctx.mem_status()[0] == two
+        # a layer's four products and the head's, per batch of 32 tokens
+        assert names[0] == 5 * ((n - 1) // 32)
+        m.close()
