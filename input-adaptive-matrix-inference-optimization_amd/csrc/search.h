@@ -392,19 +392,26 @@ __device__ __forceinline__ float search_cutoff(const float (&v)[IAM_PROBES_COUNT
 //   D. wave 0 ranks the list, or reads the fine bins from the top of the
 //      16 that hold kmin: where kmax lies within 128 of them and no bin
 //      holding a rank kmin .. kmax has more than two keys, those keys are
-//      u_kmin .. u_kmax; otherwise the keys of those fine bins are gathered
-//      (two more barriers) and ranked.  Either way u_{t-2} .. u_{t+2} come
+//      u_kmin .. u_kmax; bins of more but equal keys (many inputs 0, few
+//      distinct values) are read the same way, the last of them also past
+//      the 128; otherwise the keys of those fine bins are gathered (two more
+//      barriers; not those of an end bin of equal keys) and ranked.  Either way u_{t-2} .. u_{t+2} come
 //      out exactly, and wave 0 replays the reference's rounds from them
 //      while the other waves run the caller's `overlap(hi)` (wave 0 runs it
 //      after its tail) with hi > cutoff from the window of B (cutoff_upper),
 //      so that rows certain to be selected can be listed while the search
 //      finishes; a barrier then hands the cutoff to all.
 // It declines (in every wave at the same step) when an importance is NaN or
-// a list would be longer than kListCap; search_cutoff then finds the cutoff.  Histograms are read with one lane per NB consecutive
-// bins (NB = 32 coarse, 16 fine), stored so that a wave's 16-byte reads are
-// contiguous.
+// a list would be longer than kListCap; search_cutoff then finds the cutoff.
+// Declining late is dear: the standalone search of 4096 inputs, 19 of 20 of
+// them 0, took 22.8 us at effort 0.05 and 32.7 at 0.25 when a bin of equal
+// keys counted as a long list (the radix search alone 8.8 and 19.0), now 7.9;
+// without ties 4.7 as before.
+// Histograms are read with one lane per NB consecutive bins (NB = 32 coarse,
+// 16 fine), stored so that a wave's 16-byte reads are contiguous.
 constexpr int kCoarseBins = 2048;
 constexpr int kFineBins = 1024;
+constexpr uint32_t kKeyZero = 0x80000000u;  // the window search's key of 0, the lowest
 constexpr uint32_t kKeyInf = 0xff800000u;   // the window search's key of +inf (NaN keys lie above)
 constexpr int kListCap = 64;
 constexpr int kSmallWindow = 32;   // a window of at most this many keys is listed outright
@@ -426,6 +433,7 @@ struct WindowLds {
     // wave 0's hand-over
     int step, nl, above;
     uint32_t rlo, rhi;
+    uint32_t tie_hi, tie_lo;    // the key of every rank above the list, and below it (0: none)
     float cut;
     float hint;                 // the hinted window's centre (thread 0 stores it before a barrier)
     // hinted pass, over the waves (LDS atomics): min key, max key, keys above
@@ -446,14 +454,14 @@ __device__ __forceinline__ int hist_slot(int b)
 
 __device__ __forceinline__ int coarse_bin(uint32_t key) { return (int)((key >> 20) & (kCoarseBins - 1)); }
 
-// A key added to fine bin b < kFineBins (its count, largest and smallest
-// key).  The byte offset of hist_slot<16>(b) as three bit fields: bits 0-1
+// A key added n times to fine bin b < kFineBins (its count, largest and
+// smallest key).  The byte offset of hist_slot<16>(b) as three bit fields: bits 0-1
 // of b move to 2-3, bits 2-3 to 10-11, bits 4-9 stay.
 template <int NW>
-__device__ __forceinline__ void fine_add(WindowLds<NW>& W, uint32_t b, uint32_t key)
+__device__ __forceinline__ void fine_add(WindowLds<NW>& W, uint32_t b, uint32_t key, uint32_t n = 1u)
 {
     const uint32_t off = (b & 0x3f0u) | ((b << 2) & 0xcu) | ((b << 8) & 0xc00u);
-    atomicAdd(reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(W.fine) + off), 1u);
+    atomicAdd(reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(W.fine) + off), n);
     atomicMax(reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(W.fmax) + off), key);
     atomicMax(reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(W.fminv) + off), ~key);
 }
@@ -543,13 +551,17 @@ __device__ __forceinline__ void read_ukeys(const WindowLds<NW>& W, float (&U)[5]
 }
 
 // wave 0: u_{t-2} .. u_{t+2} from the nl listed keys: lane i's key holds
-// ranks above + gt + 1 .. above + ge
+// ranks above + gt + 1 .. above + ge.  The ranks above the list have the key
+// tie_hi, those below it tie_lo (0: none of the five lies there).
 template <int NW>
-__device__ __forceinline__ void rank_list(WindowLds<NW>& W, int nl, int above, int t, float (&U)[5])
+__device__ __forceinline__ void rank_list(WindowLds<NW>& W, int nl, int above, int t, uint32_t tie_hi, uint32_t tie_lo,
+                                          float (&U)[5])
 {
     const int lane = threadIdx.x & 63;
     const uint32_t lk = lane < nl ? W.list[lane] : 0u;
-    if (lane < 5) W.ukey[lane] = 0u;
+    const int rank = t - 2 + lane;
+    if (lane < 5)
+        W.ukey[lane] = rank <= above ? tie_hi : rank > above + nl && rank <= IAM_PROBES_COUNT ? tie_lo : 0u;
     int gt = above, ge = above;
     for (int j = 0; j < nl; j++) {
         const uint32_t kj = (uint32_t)__builtin_amdgcn_readlane((int)lk, j);
@@ -815,6 +827,20 @@ __device__ __forceinline__ int search_window(const float (&v)[IAM_PROBES_COUNT /
 #pragma unroll
             for (int k = 0; k < VPT; k++)
                 if (key[k] - base < width) W.list[atomicAdd(&W.nlist, 1u)] = key[k];
+        } else if (base == kKeyZero) {
+            // Zeros (sparse or padded inputs) meet in one bin, and adds to one
+            // address go one after the other: a wave adds its own together.
+            // (In A, too, they would be worth it, but the test for them there
+            // takes every search 0.17 us.)
+            uint32_t nz = 0u;
+#pragma unroll
+            for (int k = 0; k < VPT; k++) {
+                const uint32_t rel = key[k] - base;
+                nz += rel == 0u ? 1u : 0u;
+                if (rel != 0u && rel < width) fine_add(W, rel >> sf, key[k]);
+            }
+            nz = wave_sum(nz);
+            if (lane == 0 && nz) fine_add(W, 0u, kKeyZero, nz);
         } else {
 #pragma unroll
             for (int k = 0; k < VPT; k++) {
@@ -832,7 +858,7 @@ __device__ __forceinline__ int search_window(const float (&v)[IAM_PROBES_COUNT /
         bool rounds = true;
         if (last) {
         } else if (listed) {
-            rank_list(W, mc, ab_hi, t, U);
+            rank_list(W, mc, ab_hi, t, 0u, 0u, U);
         } else {
             // the fine bins of window ranks r1 = kmin - ab_hi .. r2 = kmax - ab_hi:
             // from the top bin of the lane whose 16 bins hold r1, lane l reads
@@ -863,17 +889,44 @@ __device__ __forceinline__ int search_window(const float (&v)[IAM_PROBES_COUNT /
                 if (c1 >= 1 && (unsigned)o1 < 5u) W.ukey[o1] = x1;
                 if (c1 == 2 && (unsigned)(o1 + 1) < 5u) W.ukey[o1 + 1] = n1;
                 read_ukeys(W, U);
-            } else {   // list the keys of the fine bins flo .. fhi
-                rounds = false;
+            } else {
                 int fhi, ab_f, flo, ab_flo, c_flo;
                 hist_find2<16>(W.fine, fs, r1, r2, fhi, ab_f, flo, ab_flo, c_flo);
-                if (lane == 0) {
-                    const int nl = ab_flo + c_flo - ab_f;
-                    W.step = nl > kListCap ? kWinDecline : kWinList;
-                    W.nl = nl;
-                    W.above = ab_hi + ab_f;
-                    W.rlo = (uint32_t)flo << sf;
-                    W.rhi = min((uint32_t)(fhi + 1) << sf, width);
+                // a bin whose largest key is its smallest holds equal keys
+                const int sh = hist_slot<16>(fhi), sl = hist_slot<16>(flo);
+                const uint32_t kh = W.fmax[sh], kl = W.fmax[sl];
+                const bool eh = kh == ~W.fminv[sh], el = kl == ~W.fminv[sl];
+                const int reach = a1 + __builtin_amdgcn_readlane(incl, 63);   // window keys down to the 128th bin
+                const bool mixed = (ov0 && c0 > 2 && x0 != n0) || (ov1 && c1 > 2 && x1 != n1);
+                if (__ballot(mixed) == 0ull && (reach >= r2 || (el && ab_flo <= reach))) {
+                    // read like the direct ones: a bin's first rank has its
+                    // largest key, its others the smallest; past the 128 bins
+                    // the equal keys of the last one
+                    const int rank = t - 2 + lane;
+                    if (lane < 5) W.ukey[lane] = rank - ab_hi > reach && rank <= IAM_PROBES_COUNT ? kl : 0u;
+#pragma unroll
+                    for (int o = 0; o < 5; o++) {
+                        const int k = t - 2 + o - ab_hi;
+                        if (e0 < k && k <= e0 + c0) W.ukey[o] = k == e0 + 1 ? x0 : n0;
+                        if (e1 < k && k <= e1 + c1) W.ukey[o] = k == e1 + 1 ? x1 : n1;
+                    }
+                    read_ukeys(W, U);
+                } else {
+                    // list the keys of the fine bins flo .. fhi, but for an end
+                    // bin of equal keys (where both ends are one such bin, the
+                    // list is empty: every rank asked for lies "above" it)
+                    rounds = false;
+                    if (lane == 0) {
+                        const int top_f = eh ? ab_f + (int)W.fine[sh] : ab_f;   // window keys above the list
+                        const int nl = max(0, (el ? ab_flo : ab_flo + c_flo) - top_f);
+                        W.step = nl > kListCap ? kWinDecline : kWinList;
+                        W.nl = nl;
+                        W.above = ab_hi + top_f;
+                        W.rlo = (uint32_t)(el ? flo + 1 : flo) << sf;
+                        W.rhi = min((uint32_t)(eh ? fhi : fhi + 1) << sf, width);
+                        W.tie_hi = eh ? kh : 0u;
+                        W.tie_lo = el ? kl : 0u;
+                    }
                 }
             }
         }
@@ -900,7 +953,7 @@ __device__ __forceinline__ int search_window(const float (&v)[IAM_PROBES_COUNT /
     __syncthreads();
     if (wave == 0) {
         float U[5];
-        rank_list(W, W.nl, W.above, t, U);
+        rank_list(W, W.nl, W.above, t, W.tie_hi, W.tie_lo, U);
         window_finish(W, U, t, kmn, kmx);
     }
     __syncthreads();

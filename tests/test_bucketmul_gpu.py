@@ -39,9 +39,9 @@ def rel_l2(a, b):
 
 
 def run_gpu(ctx, b, s, p, x, effort, in_size=None, expert_no=0, expert_rows=None, split=True, fused=None):
-    """split: calc_dispatch + mul; else full_mul (both with the cutoff
-    launch); fused (the iam module): the walk computes the cutoff itself
-    (iam_bucketmul_fused)."""
+    """split: calc_dispatch + mul (the cutoff in a launch of its own); else
+    full_mul, or, with fused (the iam module), iam_bucketmul_fused (both: the
+    walk computes the cutoff itself)."""
     R = expert_rows if expert_rows is not None else b.shape[0]
     C = b.shape[1]
     in_size = in_size if in_size is not None else R // 16
@@ -163,9 +163,8 @@ def _cutoff_patterns():
 @pytest.mark.parametrize("pattern", [p[0] for p in _cutoff_patterns()])
 def test_cutoff_edge_paths(O, iam, ctx, pattern):
     """The search's edge paths on the GPU, bit-exact against the oracle: the
-    standalone cutoff kernel (calc_dispatch + mul, 4 waves, 16 importances
-    per thread), and the walk's own search (iam_bucketmul_fused, 8 waves, 8
-    per thread) on a 256-output matrix and on the LM-head shape."""
+    standalone cutoff kernel (calc_dispatch + mul) and the walk's own search
+    (iam_bucketmul_fused) on a 256-output matrix and on the LM-head shape."""
     name, x, effort, (rounds, conv) = next(p for p in _cutoff_patterns() if p[0] == pattern)
     probes = np.full(4096, 0x2400, np.uint16)
     _, tr = O.find_cutoff(x, probes, O.effort_quantile(effort), trace=True)
@@ -228,14 +227,14 @@ _SEARCH_KINDS = ["normal", "skew", "ties", "constant", "outlier", "tiny", "inf",
 def test_cutoff_search_kinds(O, iam, ctx, kind):
     """The cutoff search bit-exact against the oracle on 16 importance
     patterns at efforts that give the quantiles 0..3, 4092..4095 and the
-    usual ones: the standalone cutoff kernel (4 waves, radix search) and the
-    walk's own search (8 waves) on 256 and 32000 outputs; the selected row
-    count matches too.  On the walk's windowed search these patterns take
-    every route: the three smallest keys (quantile 0, effort 1), a listed
-    small window (e.g. normal at the other extreme quantiles), the fine
-    bins read directly (normal at 1023), the fine bins' keys gathered and
-    ranked (quantized at 1023), and the radix search after a decline at the
-    window (all_nan) or at the list (constant)."""
+    usual ones: the standalone cutoff kernel and the walk's own search on 256
+    and 32000 outputs; the selected row count matches too.  On the windowed
+    search these patterns take every route but two (test_cutoff_search_ties):
+    the three smallest keys (quantile 0, effort 1), a listed small window
+    (e.g. normal at the other extreme quantiles), the fine bins read directly
+    (normal at 1023), bins of equal keys read directly (constant), the fine
+    bins' keys gathered and ranked (quantized at 1023), and the radix search
+    after a decline at the window (all_nan)."""
     rng = np.random.default_rng(100 + _SEARCH_KINDS.index(kind))
     x, p = _search_input(kind, rng)
     quants = [0, 1, 2, 3, 100, 1023, 2047, 3071, 3583, 3890, 4092, 4093, 4094, 4095]
@@ -271,6 +270,52 @@ def test_cutoff_search_kinds(O, iam, ctx, kind):
         ds.free()
     dp.free()
     dx.free()
+
+
+def _tied_input(kind, rng):
+    """(x, ranks): x with groups of equal |x| (every probe is 2^-6, so equal
+    importances), and the ranks (descending, 1-based) where its groups end."""
+    def groups(values, sizes):
+        assert sum(sizes) == 4096
+        return np.repeat(np.asarray(values, np.float64), sizes), list(np.cumsum(sizes)[:-1])
+    near = 0.64 * (1 - 2.0 ** -10 - 2.0 ** -21 * np.arange(30))   # 30 keys in few fine bins
+    if kind == "sparse":                    # inputs 0 but for 1 in 20
+        v = np.where(np.arange(4096) < 205, np.abs(rng.normal(0, 1, 4096)), 0.0)
+        ends = [205]
+    elif kind == "levels":                  # 32 values of one binade
+        v, ends = groups(np.linspace(1.9, 1.0, 32), [128] * 32)
+    elif kind == "far":                     # values past 128 fine bins of each other
+        v, ends = groups([100.0, 1.0, 2.0 ** -20, 0.0], [500, 1500, 1000, 1096])
+    elif kind == "gap":                     # zeros below a dense cluster in one fine bin
+        v = np.concatenate([1.0 + rng.random(2048) * 0.01, np.zeros(2048)])
+        ends = [1000, 2048]
+    elif kind == "tie_then_mixed":
+        v, ends = groups(np.concatenate([[0.64], near, [0.1]]), [500] + [1] * 30 + [3566])
+    elif kind == "mixed_then_tie":
+        v, ends = groups(np.concatenate([[1.2], near, [0.63]]), [2000] + [1] * 30 + [2066])
+    else:                                   # single keys between two ties
+        v, ends = groups([0.64, 0.6399, 0.6398, 0.63], [1500, 1, 2, 2593])
+    return rng.permutation(v * rng.choice([-1.0, 1.0], 4096)).astype(np.float32), [int(e) for e in ends]
+
+
+@pytest.mark.parametrize("kind", ["sparse", "levels", "far", "gap", "tie_then_mixed", "mixed_then_tie", "singles"])
+def test_cutoff_search_ties(O, iam, ctx, kind):
+    """Groups of many equal importances, with the target rank on either side
+    of a group's end and inside it: bins of equal keys read directly, also
+    the last one past the 128 bins read (far, sparse), as the ends of a list
+    (tie_then_mixed, mixed_then_tie), and a decline at a list too long (gap).
+    The cutoff and the selected rows are the oracle's bit for bit in the
+    standalone search and in the walk's."""
+    rng = np.random.default_rng(500 + len(kind))
+    x, ends = _tied_input(kind, rng)
+    p = np.full(4096, 0x2400, np.uint16)
+    b, s, _ = make_matrix(O, 256, 4096, tid=9)
+    for t in sorted({e + o for e in ends[:3] + ends[-1:] for o in (-40, -3, -2, -1, 0, 1, 2, 3, 40)}):
+        q = 4096 - t
+        effort = float(np.float32(1.0 - (q + 0.5) / 4095.0))
+        assert O.effort_quantile(effort) == q
+        for kw in (dict(split=True), dict(split=False), dict(fused=iam)):
+            check_against_oracle(O, ctx, b, s, p, x, effort, **kw)
 
 
 _HINT_KINDS = ["normal", "skew", "ties", "constant", "outlier", "tiny", "inf", "nan", "huge",
