@@ -437,6 +437,18 @@ def test_long_slices(O, iam, ctx, out_dim, effort):
     check_against_oracle(O, ctx, b[:4000 * 16], s[:4000 * 16], p, x, effort, in_size=4000, expert_rows=4000 * 16)
 
 
+@pytest.mark.parametrize("out_dim", [64, 1024])
+@pytest.mark.parametrize("in_dim,effort", [(4096, 0.6), (4096, 0.7), (4096, 1.0), (8200, 0.25), (8200, 1.0)])
+def test_long_slices_many_rows(O, iam, ctx, out_dim, in_dim, effort):
+    """Few column tiles and many rows, on either side of the row count from
+    which the slices hold 512 of them (31,000 and 34,000 rows expected; 42,000
+    and more), a partial last slice among them."""
+    b, s, p = make_matrix(O, out_dim, in_dim, tid=8)
+    x = O.gen_f32(0, 11, in_dim, 0.0, 1.0)
+    for kw in (dict(split=True), dict(split=False), dict(fused=iam)):
+        check_against_oracle(O, ctx, b, s, p, x, effort, **kw)
+
+
 def test_in_size_skips_rows(O, ctx):
     b, s, p = make_matrix(O, 256, 4096, tid=13)
     x = O.gen_f32(0, 14, 4096, 0.0, 1.0)
