@@ -85,6 +85,29 @@ def test_gpu_bucketizer_edges(O, ctx, shape):
     assert np.array_equal(b, ob.ravel()) and np.array_equal(s, os_.ravel()) and np.array_equal(p, op)
 
 
+# every bucket count below 8 and the first one past it; one input, and the
+# ends of the 64-input workgroups
+@pytest.mark.parametrize("shape", [(16, 4097), (32, 64), (48, 1), (64, 63), (80, 130), (96, 65), (112, 1000), (128, 100)])
+def test_gpu_bucketizer_few_buckets(O, ctx, shape):
+    """As test_gpu_bucketizer_edges, where a thread holds a whole input, into
+    buckets at a 2-byte boundary; the words on either side are left alone."""
+    W = O.gen_f16(6, 79, shape[0] * shape[1], 0.0, 0.02).reshape(shape).copy()
+    W[::7] = W[::7] & 0x8FFF
+    W[3::16, ::3] = W[2::16, ::3] ^ 0x8000
+    W[5::16, ::5] = 0x7C00
+    W[6::16, ::5] = 0xFC00
+    n = W.size
+    dw, db = ctx.upload(W), ctx.upload(np.full(n + 2, 0xABCD, np.uint16))
+    ds, dp = ctx.empty(64 * shape[1], np.uint16), ctx.empty(shape[1], np.uint16)
+    ctx.bucketize(dw, shape[0], shape[1], db.ptr + 2, ds, dp)
+    b, s, p = db.read(np.uint16), ds.read(np.uint16), dp.read(np.uint16)
+    for d in (dw, db, ds, dp):
+        d.free()
+    ob, os_, op = O.bucketize(W)
+    assert b[0] == b[-1] == 0xABCD
+    assert np.array_equal(b[1:-1], ob.ravel()) and np.array_equal(s, os_.ravel()) and np.array_equal(p, op)
+
+
 def test_rmsnorm_and_add(O, ctx):
     x = O.gen_f32(0, 31, 4096, 0.0, 1.0)
     dlt = O.gen_f32(0, 32, 4096, 0.0, 0.5)
