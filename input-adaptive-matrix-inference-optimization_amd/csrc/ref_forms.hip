@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "internal.h"
 #include "layer_ops.h"
@@ -211,12 +212,16 @@ __global__ __launch_bounds__(kHD) void k_att32_sum(const int* __restrict__ pos_p
 // between lanes 32 .. 1 apart, strides 2 and 1 stay in lane 0.  x is staged
 // in LDS; each wave walks rows wave, wave + waves, ... two at a time, eight
 // loads of a row in flight (32000 x 4096: 64.8 us with the loads the compiler
-// left between the adds, 46 with these, 5.7 TB/s).
+// left between the adds, 42 with these, 6.2 TB/s), and of a shorter row or
+// rest its 4, 2 and 1 blocks together, the partial one's first (32000 x 1024
+// and 1000: 32 and 33 us with a loop over single blocks behind the eights, 21
+// where that loop stood alone, 16 and 19 with these).  5 waves a SIMD: one
+// more in flight than the compiler's choice (45 us for 32000 x 4096).
 constexpr int kDenseThreads = 256;
 constexpr int kDenseMaxCols = 16384;
 
 template <bool VEC>
-__global__ __launch_bounds__(kDenseThreads) void k_matmul16x32(const uint16_t* __restrict__ W,
+__global__ __launch_bounds__(kDenseThreads, 5) void k_matmul16x32(const uint16_t* __restrict__ W,
                                                                const float* __restrict__ x, int rows, int cols,
                                                                float* __restrict__ out)
 {
@@ -233,38 +238,43 @@ __global__ __launch_bounds__(kDenseThreads) void k_matmul16x32(const uint16_t* _
 #pragma unroll
         for (int c = 0; c < 4; c++) s[c] = 0.0f;
         int k = 0;
-        // whole columns blocks: 8 loads in flight a row, added in order
+        // Whole columns blocks: 8 loads in flight a row, added in order, then
+        // the 4, 2 and 1 of what is left; a partial block's load goes out
+        // ahead of them all.
         if constexpr (VEC) {
             typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-            for (; (k + 8) * kDenseWG <= cols; k += 8) {
-                u32x2 p[8];
+            auto load = [&](int b) { return __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(w + b)); };
+            auto add = [&](const u32x2& p, int b) {
+                const float4 xv = *reinterpret_cast<const float4*>(sx + b);
+                s[0] = __fadd_rn(s[0], __fmul_rn(f16(p.x), xv.x));
+                s[1] = __fadd_rn(s[1], __fmul_rn(f16(p.x >> 16), xv.y));
+                s[2] = __fadd_rn(s[2], __fmul_rn(f16(p.y), xv.z));
+                s[3] = __fadd_rn(s[3], __fmul_rn(f16(p.y >> 16), xv.w));
+            };
+            auto blocks = [&](auto n_tag) {
+                constexpr int N = decltype(n_tag)::value;
+                u32x2 p[N];
 #pragma unroll
-                for (int u = 0; u < 8; u++)
-                    p[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(w + (k + u) * kDenseWG + 4 * lane));
+                for (int u = 0; u < N; u++) p[u] = load((k + u) * kDenseWG + 4 * lane);
 #pragma unroll
-                for (int u = 0; u < 8; u++) {
-                    const float4 xv = *reinterpret_cast<const float4*>(sx + (k + u) * kDenseWG + 4 * lane);
-                    s[0] = __fadd_rn(s[0], __fmul_rn(f16(p[u].x), xv.x));
-                    s[1] = __fadd_rn(s[1], __fmul_rn(f16(p[u].x >> 16), xv.y));
-                    s[2] = __fadd_rn(s[2], __fmul_rn(f16(p[u].y), xv.z));
-                    s[3] = __fadd_rn(s[3], __fmul_rn(f16(p[u].y >> 16), xv.w));
-                }
-            }
+                for (int u = 0; u < N; u++) add(p[u], (k + u) * kDenseWG + 4 * lane);
+                k += N;
+            };
+            const int whole = cols / kDenseWG, last = whole * kDenseWG + 4 * lane;
+            u32x2 part{};
+            if (last < cols) part = load(last);
+            while (k + 8 <= whole) blocks(std::integral_constant<int, 8>{});
+            if (k + 4 <= whole) blocks(std::integral_constant<int, 4>{});
+            if (k + 2 <= whole) blocks(std::integral_constant<int, 2>{});
+            if (k < whole) blocks(std::integral_constant<int, 1>{});
+            if (last < cols) add(part, last);
+            return;
         }
         for (; k < nk; k++) {
             const int b = k * kDenseWG + 4 * lane;
             uint32_t v[4];
-            if (VEC && b + 3 < cols) {
-                typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-                const u32x2 p = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(w + b));
-                v[0] = p.x;
-                v[1] = p.x >> 16;
-                v[2] = p.y;
-                v[3] = p.y >> 16;
-            } else {
 #pragma unroll
-                for (int c = 0; c < 4; c++) v[c] = b + c < cols ? (uint32_t)w[b + c] : 0u;
-            }
+            for (int c = 0; c < 4; c++) v[c] = b + c < cols ? (uint32_t)w[b + c] : 0u;
 #pragma unroll
             for (int c = 0; c < 4; c++)
                 if (b + c < cols) s[c] = __fadd_rn(s[c], __fmul_rn(f16(v[c]), sx[b + c]));

@@ -165,6 +165,15 @@ def test_matmul_f16_dense_eight_blocks(O, ctx, rows, cols):
     test_matmul_f16_dense_bit_exact(O, ctx, rows, cols)
 
 
+@pytest.mark.parametrize("rows,cols", [(5, 4), (3, 252), (9, 260), (4, 1000), (33, 1024), (2, 1284), (7, 1792), (1, 2040),
+                                       (3, 3844), (2, 16384), (2, 1001)])
+def test_matmul_f16_dense_rest_of_a_row(O, ctx, rows, cols):
+    """Bit-exact with every rest of whole blocks (1 to 7) behind the eights or
+    alone, with a partial block and without, and columns that are no multiple
+    of 4."""
+    test_matmul_f16_dense_bit_exact(O, ctx, rows, cols)
+
+
 @pytest.mark.parametrize("n", [1, 1023, 1025, 16384, 16385, 40001])
 def test_argmax_rounds(O, ctx, n):
     """The first maximum at the ends of the threads' rounds of 16 values, with
