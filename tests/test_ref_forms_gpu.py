@@ -187,3 +187,11 @@ def test_argmax_rounds(O, ctx, n):
         assert di.read()[0] == at[0]
         dv.free()
         di.free()
+
+
+@pytest.mark.parametrize("rounds", [1, 2, 3, 4, 5, 8, 9, 16, 17, 20, 25, 32])
+def test_argmax_last_rounds(O, ctx, rounds):
+    """Every number of values a thread has left (1, 2, 4, 8 and 16 at a time):
+    a whole last round, all but one value of it, and its first value only."""
+    for n in (rounds * 1024, rounds * 1024 - 1, rounds * 1024 - 1023):
+        test_argmax_rounds(O, ctx, n)
