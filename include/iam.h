@@ -378,7 +378,7 @@ int iam_model_step_device(iam_model* m, float effort, const float* hidden_overri
  * generates n_new tokens with first-max argmax.  With use_graph the per-token
  * step is captured once as a HIP graph and replayed.  The prompt's tokens
  * before the last go through the model in batches where that is faster (fp64
- * accumulation, from 8 to 16 tokens on by effort), in buffers the model keeps
+ * accumulation, from 6 to 16 tokens on by shape and effort), in buffers the model keeps
  * until an allocation needs their room (about 2 MB a token, at most 512
  * tokens', at 4096 wide with FFN 14336; fewer where there is less room); the
  * KV cache, the picks in "history" and the walk counters are as by steps, and

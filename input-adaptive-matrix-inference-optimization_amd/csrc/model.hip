@@ -459,19 +459,48 @@ static int run_steps(iam_model* m, int n, float effort, bool use_graph)
     return IAM_OK;
 }
 
-// How many of `tokens` (up to a chunk) the batched prefill takes; the decode
-// step does the others faster.  A step's time grows with the share of rows the
-// effort selects, a batch's with its groups of 16 tokens whatever the effort.
-// Measured on 4 layers and the LM head, 4096 wide with FFN 14336, a token by
-// steps against the first group: 0.245, 0.29 and 0.51 ms at efforts 0.05, 0.25
-// and 1.0 against 3.85 ms (equal at 15.7, 13.3 and 7.5 tokens); each further
-// group takes 1.3 ms, a third of that.
-static int pf_take(int tokens, float effort)
+// Estimated times, in ms, that decide between batches and steps; gw: billions
+// of weights.  A step: its launches, then the selected bytes (a fit of decode
+// runs over layers, widths and efforts).  A batch costs the same at every
+// effort: its launches, and by the workgroup rows of the products, which hold
+// 1, 2 or 4 groups of 16 tokens; past 4 groups each further 1 to 4 of them
+// open a whole row.  Measured in a batch of 1, 2, 3-4, 5-8, 9-12 and 13-16
+// groups: 4 layers 4096 wide with FFN 14336 and a head of 32000 (1.0 billion)
+// 3.6, 4.9, 7.7, 12.4, 17.9 and 23.5 ms, a step 0.245, 0.29 and 0.51 ms at
+// efforts 0.05, 0.25 and 1.0; 2 layers with FFN 4096 and a head of 512 (0.19
+// billion) 1.0, 1.3, 1.9, 2.8, 3.9 and 5.0, a step 0.127, 0.136 and 0.166.  With
+// 71 tokens the first of these takes 64 in a batch and 6 by steps, 9.5, 9.8
+// and 11.4 ms (all in a batch 12.5 to 12.8).
+static double pf_step_ms(double gw, int layers, float effort)
 {
-    const double scale = 1.0 + 1.4 * est_rows(1 << 20, effort) / (1 << 20);
-    const int rest = tokens % kPfGroup, whole = tokens - rest;
-    if (whole == 0) return rest >= 18.0 / scale ? rest : 0;
-    return rest >= 6.0 / scale ? tokens : whole;
+    return 0.02 + 0.051 * layers + 0.30 * gw * est_rows(1 << 20, effort) / (1 << 20);
+}
+
+static double pf_batch_ms(double gw, int layers, int groups)
+{
+    const double products = groups == 1 ? 2.85 : groups == 2 ? 4.15 : 7.0 + 5.2 * ((groups + 3) / 4 - 1);
+    return 0.12 + 0.18 * layers + products * gw;
+}
+
+// How many of `tokens` (up to a chunk) the batched prefill takes; the decode
+// step does the others faster.
+static int pf_take(const iam_model* m, int tokens, float effort)
+{
+    const iam_model_config& C = m->cfg;
+    const double D = C.dim, KVD = (double)C.n_kv_heads * C.head_dim;
+    const double gw = 1e-9 * D * (C.n_layers * (2.0 * D + 2.0 * KVD + 3.0 * C.ffn_dim) + (m->lm_dense ? 0.0 : C.vocab));
+    const double step = pf_step_ms(gw, C.n_layers, effort);
+    int best = 0;
+    double least = tokens * step;
+    for (int g = 1; g <= pf_groups(tokens); g++) {
+        const int t = std::min(tokens, g * kPfGroup);
+        const double ms = pf_batch_ms(gw, C.n_layers, g) + (tokens - t) * step;
+        if (ms < least) {
+            least = ms;
+            best = t;
+        }
+    }
+    return best;
 }
 
 // The buffers of one prefill chunk, laid out in pf.p.
@@ -623,11 +652,11 @@ static int pf_chunk(iam_model* m, const PfBuffers& B, int pos0, int tokens, floa
 static int prefill_batched(iam_model* m, const int* prompt, int n, float effort, int* done)
 {
     *done = 0;
-    const int largest = pf_take(std::min(n, kPfMaxTokens), effort);
+    const int largest = pf_take(m, std::min(n, kPfMaxTokens), effort);
     if (largest == 0 || !m->c->acc64 || !pf_ensure(m, largest)) return IAM_OK;
     const int most = std::min(kPfMaxTokens, m->pf.cap);
     while (*done < n) {
-        const int chunk = std::min(n - *done, most), tokens = pf_take(chunk, effort);
+        const int chunk = std::min(n - *done, most), tokens = pf_take(m, chunk, effort);
         if (tokens == 0) break;
         PfBuffers B;
         (void)pf_layout(m, tokens, m->pf.p, &B);

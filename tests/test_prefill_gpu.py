@@ -86,6 +86,14 @@ def test_token_groups(O, ctx, model, n, effort):
     check(O, ctx, model, BASE, n, effort)
 
 
+# the tokens past a multiple of 64: all in the batch, or the ones past the last
+# full group, or all of them by steps (which of these, the effort decides)
+@pytest.mark.parametrize("n", [66, 68, 75, 82, 98, 122])
+@pytest.mark.parametrize("effort", [0.05, 1.0])
+def test_tokens_past_a_row(O, ctx, model, n, effort):
+    check(O, ctx, model, BASE, n, effort)
+
+
 @pytest.mark.parametrize("kw,n", [(dict(ffn_dim=4112, vocab=528), 40),                 # 257 and 33 bucket columns
                                   (dict(dim=5120, n_heads=40, n_kv_heads=8, n_layers=1), 20),   # the norm apart
                                   (dict(ffn_dim=5008, n_kv_heads=4, vocab=16, n_layers=1), 70)])
