@@ -202,7 +202,11 @@ __device__ __forceinline__ void fma_below(double& acc, double w, uint32_t rank, 
 }
 
 // A vector instruction's write of exec wants 4 wait states before a lane read
-// or write; the compiler, which spills scalars with those, sees none in the asm
+// or write (5 before a DPP operand).  The compiler sees no such write in the
+// asm, and it spills scalars with lane writes.  This stands after a run of
+// fma_below; within the run nothing but scalar arithmetic may fall between
+// them, which the source cannot say: tests/test_prefill_asm.py reads the
+// assembly for it.
 __device__ __forceinline__ void exec_settled() { asm volatile("s_nop 3"); }
 
 template <int WT>
