@@ -106,6 +106,77 @@ def test_ragged_shapes(O, iam, ctx, kw, n):
         m.close()
 
 
+# (two layers: the second one's cache depends on the first one's attention)
+LONG = dict(BASE, n_kv_heads=32, max_ctx=1152)
+
+
+@pytest.fixture(scope="module")
+def long_model(iam, ctx):
+    """One query head per KV head (attention's one-head form) and room for
+    prompts of more than two chunks of 512."""
+    m = make(iam, ctx, n_kv_heads=32, max_ctx=1152)
+    yield m
+    m.close()
+
+
+# one chunk past 64 and past 128 positions; a second chunk the steps take (4
+# tokens), a batch takes (47, part of a group), in part (70); three chunks; the
+# whole KV capacity
+@pytest.mark.parametrize("n,effort", [(100, 0.25), (200, 0.05), (517, 0.25), (560, 0.25), (583, 0.05), (1050, 1.0),
+                                      (1151, 0.25)])
+def test_prompts_of_several_chunks(O, ctx, long_model, n, effort):
+    check(O, ctx, long_model, LONG, n, effort)
+
+
+def test_several_chunks_pair_heads_and_batches(O, iam, ctx):
+    """Two heads per workgroup, and the number of batches that run."""
+    cfg = dict(BASE, max_ctx=640)
+    m = make(iam, ctx, max_ctx=640)
+    try:
+        names = []
+
+        def batches():
+            ctx.sync()
+            ctx.profiling(False)
+            names.append(ctx.kernel_stat("prefill.pick")[1])
+
+        ctx.kernel_stats_reset()
+        ctx.profiling(True)
+        check(O, ctx, m, cfg, 560, 0.25, after=batches)
+        assert names == [2]
+    finally:
+        ctx.profiling(False)
+        m.close()
+
+
+def test_several_chunks_dense_head(O, iam, ctx, long_model):
+    """The dense head's picks and the cache of a prompt of two chunks."""
+    head = ctx.upload(O.gen_f16(0, 21, 512 * 4096, 0.0, 0.02))
+    n = 600
+    prompt = O.gen_tokens(0, 8, n, 512)
+    long_model.set_lm_dense(head)
+    try:
+        long_model.reset_caches()
+        got = long_model.generate(prompt, 1, 0.25)
+        k, v, hist, _ = state(long_model, LONG, n)
+        long_model.reset_caches()
+        log = ctx.empty(512, np.float32)
+        picks = []
+        for pos, tok in enumerate(prompt):
+            long_model.forward(int(tok), pos, 0.25, log)
+            picks.append(O.argmax(log.read()))
+        wk, wv, _, _ = state(long_model, LONG, n)
+        log.free()
+        for a, b in ((k, wk), (v, wv)):
+            d = ulp16(a, b)
+            assert np.mean(d != 0) < 1e-3 and d.max() <= 1
+        assert np.mean(hist != np.array(picks)) <= 0.02
+        assert got[0] == hist[-1]
+    finally:
+        long_model.set_lm_dense(None)
+        head.free()
+
+
 def test_weights_no_converter_writes(O, iam, ctx):
     """Stats that rise with the rank (the selected ranks are not the first
     ones), buckets with a position twice, and an embedding scale."""
