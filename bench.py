@@ -4,7 +4,7 @@
 Workload: 32 layers, dim 4096, FFN 14336, 32 query / 8 KV heads of 128,
 vocabulary 32000 with a bucket-layout LM head, fp16 GQA KV cache of 4096
 positions, RoPE theta 10000; random-init synthetic weights N(0, 0.02^2)
-bucketized on the GPU; a 512-token random-id prompt fed; then
+bucketized on the GPU; a 512-token random-id prompt; then
 greedy decode at effort 0.25.  A step is one decode token (captured once as a
 HIP graph and replayed).  `value` is decode tokens per second, timed with
 the library's walk counting switched off; the bytes per token come from
@@ -249,9 +249,10 @@ def config1(iam, ctx, effort, reps):
     """One 4096x4096 bucketMul at the given effort, W ~ N(0, 0.02^2)
     bucketized on the GPU, x ~ N(0, 1), seed 0.  Timed as the decode step
     runs a matrix group (iam_bucketmul_fused: input, cutoff, selection and
-    walk in one launch) and as the reference's calcDispatch + mul (multi: a
-    cutoff launch, then the walk).  CONFIG1_COPIES copies of the bucketized
-    matrix are used in turn, so none is in the Infinity Cache when it is
+    walk in one launch) and as the reference's calcDispatch + mul (a cutoff
+    launch, then the walk, over the reference's 4-channel stats).
+    CONFIG1_COPIES copies of the bucketized matrix and its stats are used in
+    turn, so none is in the Infinity Cache when it is
     read again; kernel durations come from per-dispatch events.  Bytes per
     call: 2*S*C + 2*R + 4*in + 2*4096 + 4*m (selected rows, one stats value
     per row, x, probes, y)."""
@@ -265,10 +266,12 @@ def config1(iam, ctx, effort, reps):
     b0, s0, p0 = ctx.empty(R * C, u16), ctx.empty(R * 4, u16), ctx.empty(in_dim, u16)
     ctx.bucketize(W, out_dim, in_dim, b0, s0, p0)
     s3 = ctx.stats_compact(s0, R)
-    mats, bufs = [], [W, b0, s0, p0, s3]
+    mats, stats4, bufs = [], [], [W, b0, s0, p0, s3]
     for k in range(CONFIG1_COPIES):
         b, st, pr = ctx.empty(R * C, u16), ctx.empty(R, u16), ctx.empty(in_dim, u16)
+        stats4.append(ctx.empty(R * 4, u16))
         ctx.copy(b, b0, R * C * 2)
+        ctx.copy(stats4[-1], s0, R * 8)
         ctx.copy(st, s3, R * 2)
         ctx.copy(pr, p0, in_dim * 2)
         bufs += [b, st, pr]
@@ -276,20 +279,22 @@ def config1(iam, ctx, effort, reps):
     y = ctx.empty(out_dim, np.float32)
     res = {}
     for mode in ("fused", "cutoff_launch"):
-        def call(m):
+        def call(k):
+            m = mats[k]
             if mode == "fused":
                 ctx.fused([m], x, in_dim, [y], effort)
             else:
-                ctx.multi([m], [x], [in_dim], [y], effort)
-        for m in mats:
-            call(m)
+                ctx.calc_dispatch(x, stats4[k], m.probes, 0, in_dim, C, R, effort)
+                ctx.mul(m.buckets, C, y)
+        for k in range(CONFIG1_COPIES):
+            call(k)
         ctx.sync()
         ctx.set_walk_counting(True)
         ctx.walk_counters(reset=True)
         ctx.kernel_stats_reset()
         ctx.profiling(True)
         for r in range(reps):
-            call(mats[r % CONFIG1_COPIES])
+            call(r % CONFIG1_COPIES)
         ctx.sync()
         ctx.profiling(False)
         _, rows, _ = ctx.walk_counters(reset=True)
@@ -307,7 +312,7 @@ def config1(iam, ctx, effort, reps):
                          bytes_per_call=round(B), achieved_GBs=round(gbs, 1), frac=round(gbs / HBM_PEAK_GBS, 4))
         log(f"config 1, {mode}: {t_ms * 1e3:.2f} us per call ({parts}), S = {S:.0f}, "
             f"{B / 1e6:.2f} MB -> {gbs:.0f} GB/s")
-    for d in bufs + [x, y]:
+    for d in bufs + stats4 + [x, y]:
         d.free()
     return res
 
