@@ -129,9 +129,10 @@ int iam_bucketmul_mul(iam_ctx* ctx, const uint16_t* buckets_dev, int bucket_cols
 int iam_bucketmul_full(iam_ctx* ctx, const float* x_dev, const uint16_t* stats_dev,
                        const uint16_t* probes_dev, const uint16_t* buckets_dev, int expert_no,
                        int in_size, int bucket_cols, int expert_size, float effort, float* y_dev);
-/* Up to 3 independent matrices in one cutoff launch and one walk launch
- * (the q/k/v and gate/up calls of attention.hpp:160-170 and
- * feedforward.hpp:60-68 share an input).  xs[i] may repeat. */
+/* Up to 3 independent matrices in one launch, like iam_bucketmul_full every
+ * walk workgroup running the cutoff search of its matrix itself (the q/k/v and
+ * gate/up calls of attention.hpp:160-170 and feedforward.hpp:60-68 share an
+ * input).  xs[i] may repeat. */
 int iam_bucketmul_multi(iam_ctx* ctx, int n, const iam_bucket_matrix* mats,
                         const float* const* xs_dev, const int* in_sizes, float* const* ys_dev,
                         int expert_no, float effort);
@@ -378,11 +379,13 @@ int iam_model_step_device(iam_model* m, float effort, const float* hidden_overri
  * generates n_new tokens with first-max argmax.  With use_graph the per-token
  * step is captured once as a HIP graph and replayed.  The prompt's tokens
  * before the last go through the model in batches where that is faster (fp64
- * accumulation, from 6 to 16 tokens on by shape and effort), in buffers the model keeps
- * until an allocation needs their room (about 2 MB a token, at most 512
- * tokens', at 4096 wide with FFN 14336; fewer where there is less room); the
- * KV cache, the picks in "history" and the walk counters are as by steps, and
- * the last token's step leaves the activations and logits.
+ * accumulation, from 6 to 16 tokens on by shape and effort), in buffers the
+ * model keeps until an allocation needs their room (about 2 MB a token, at
+ * most 512 tokens', at 4096 wide with FFN 14336; fewer where there is less
+ * room).  The KV cache, the picks in "history" and the walk counters' bytes,
+ * rows and matrices are as by steps; batched tokens take no search hints, so
+ * they count no tries or hits of them (iam_walk_group_hints).  The last
+ * token's step leaves the activations and logits.
  * out_tokens receives n_new ids. */
 int iam_model_generate(iam_model* m, const int* prompt, int n_prompt, int n_new, float effort,
                        int use_graph, int* out_tokens);

@@ -1298,8 +1298,8 @@ static double est_fraction(float effort)
 
 double est_rows(int rows, float effort) { return std::max(1.0, rows * est_fraction(effort)); }
 
-// Walk launch shape: 8-wave workgroups (each CU holds one: 128 KB of fp64
-// tiles), about IAM_WALK_WGS of them, shared among the matrices in
+// Walk launch shape: 8-wave workgroups (57 KB of LDS, 33 KB of it fp64 tiles;
+// a CU's registers hold one), about IAM_WALK_WGS, shared among the matrices in
 // proportion to their expected weight bytes (at least one slice each), so
 // that no CU holds more work than another.  IAM_WALK_UNR loads of RPI rows
 // form a batch, two batches in flight per wave: with 2, each batch's LDS
@@ -1678,8 +1678,9 @@ int bucketmul_walk(Ctx* c, int n, const MatOp* ops)
 // from) instead of waiting for a search launch of one workgroup per matrix.
 // The search inside the walk costs it about 3.5 us; the launch it replaces
 // took 6-8 us plus the gap between the two (1024 x 4096 at effort 0.25: 18.7
-// us a call before, 15.8 now; a 4096-wide layer of four such calls at effort
-// 0.25: 102.5 -> 85.4 us).
+// us a call with two launches, 15.8 with one, 12.0 with the slices of
+// slice_rows; a 4096-wide layer of four such calls at effort 0.25: 102.5 ->
+// 85.4 us).
 static int bucketmul_whole(Ctx* c, int n, const MatOp* ops, int expert_no, float effort)
 {
     CutoffArgs args{};

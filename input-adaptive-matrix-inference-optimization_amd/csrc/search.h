@@ -33,7 +33,7 @@
 
 namespace iam {
 
-constexpr int kCutThreads = 256;              // threads of the standalone cutoff kernels
+constexpr int kCutThreads = 256;              // threads of the list kernel (k_dispatch), with a search of its own
 constexpr int kCutVPT = IAM_PROBES_COUNT / kCutThreads;   // 16 importances per thread there
 
 template <int NW>
