@@ -85,12 +85,14 @@ def test_gpu_bucketizer_edges(O, ctx, shape):
     assert np.array_equal(b, ob.ravel()) and np.array_equal(s, os_.ravel()) and np.array_equal(p, op)
 
 
-# every bucket count below 8 and the first one past it; one input, and the
-# ends of the 64-input workgroups
-@pytest.mark.parametrize("shape", [(16, 4097), (32, 64), (48, 1), (64, 63), (80, 130), (96, 65), (112, 1000), (128, 100)])
+# every bucket count below 8, one input, the ends of the 64-input workgroups;
+# past it, in the one-pass kernel, one input and a ragged last workgroup
+@pytest.mark.parametrize("shape", [(16, 4097), (32, 64), (48, 1), (64, 63), (80, 130), (96, 65), (112, 1000), (128, 1),
+                                   (128, 17), (144, 100)])
 def test_gpu_bucketizer_few_buckets(O, ctx, shape):
-    """As test_gpu_bucketizer_edges, where a thread holds a whole input, into
-    buckets at a 2-byte boundary; the words on either side are left alone."""
+    """As test_gpu_bucketizer_edges, where a thread holds a whole input and just
+    past there, into buckets at a 2-byte boundary; the words on either side are
+    left alone."""
     W = O.gen_f16(6, 79, shape[0] * shape[1], 0.0, 0.02).reshape(shape).copy()
     W[::7] = W[::7] & 0x8FFF
     W[3::16, ::3] = W[2::16, ::3] ^ 0x8000
