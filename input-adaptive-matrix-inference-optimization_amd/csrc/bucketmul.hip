@@ -1325,14 +1325,17 @@ int sel_block_for(const Ctx* c, float effort) { return c->sel_block > 1 && effor
 // 11.5, 11.8 and 12.3.  With one to three columns a wave's load has few
 // lanes' worth of columns: 16 x 4096 12.4, 10.8 and (256) 12.1.  A decode step
 // without a finalize: 4 layers at effort 0.05 235.3 us at 1, 233.4 at 192, 235.9
-// at 256 (no change from effort 0.25 on, whose slices are longer).
+// at 256 (no change from effort 0.25 on, whose slices are longer); with inputs
+// selected in blocks of 16, which takes many more rows than the estimate, three
+// layers at effort 0.05 282.0 us at 1, 289.4 at 192 (FFN 4096: 228.7, 242.4).
 // With many rows the best slices are longer (the walk's time falls with the
 // slices' number, the queue of their adds grows with it): at 256, 384, 512
 // and 768 rows, 1024 x 4096 at effort 0.5 (26,000 rows) takes 12.3, 12.1, 12.4
 // and 13.8 us, at 0.75 (46,000) 13.7, 13.1, 12.8 and 13.0, at 1.0 16.1, 13.2,
 // 12.5 and 12.5; 1024 x 14336 at 0.25 (54,000) 15.0, 13.9, 13.5 and 13.9.
-static double slice_rows(int cols, bool finalize, double rows)
+static double slice_rows(int cols, bool finalize, double rows, int blk)
 {
+    if (!finalize && blk > 1) return 1.0;
     if (cols < 4) return 128.0;
     return !finalize ? 192.0 : rows > 36000.0 ? 512.0 : 256.0;
 }
@@ -1354,7 +1357,7 @@ void plan_walk(int n, const MatOp* ops, float effort, WalkPlan* plan, int blk, i
         pl.NW = kWalkWaves;
         const double wgs = tot > 0 ? IAM_WALK_WGS * bytes[i] / tot : (double)IAM_WALK_WGS / n;
         const double rows = est_rows(pl.n_in * 16, effort);
-        const double full = rows / slice_rows(ops[i].mat.bucket_cols, finalize, rows);
+        const double full = rows / slice_rows(ops[i].mat.bucket_cols, finalize, rows, blk);
         const int slices = std::max(1, (int)std::floor(std::min(wgs / pl.T + 1e-9, full)));
         pl.IPS = std::min(64 * pl.NW, std::max(1, (pl.n_in + slices - 1) / slices));
         if (blk > 1) pl.IPS = std::min(64 * pl.NW, (pl.IPS + blk - 1) / blk * blk);   // blocks within a slice
